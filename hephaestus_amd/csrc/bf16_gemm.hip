@@ -5,6 +5,20 @@
 // `linear`, src/hephaestus/kernels.mojo:108-118), e.g. the lm_head over
 // every position of a prompt. Rows up to 32 take the weight-streaming
 // kernel in bf16_skinny.hip.
+//
+// The DMA-staged tiles of gemm_big.h and gemm_ring.h in their bf16 form take
+// every call whose operands' byte offsets fit 32 bits: no per-chunk scales,
+// so the MFMAs accumulate in place. They are bound by the weight stream (up
+// to M of about 100) or by the MFMAs; what costs beside that is rows of the
+// last tile past M, a last round of tiles that leaves CUs idle, and the DMA's
+// latency at the start of each tile, which the choice of tile trades against
+// each other (kBf16Tiles). MI355X, graph-replayed over HBM-streamed weights,
+// against the register-staged kernel below: the lm_head (151936 x 2560, f32
+// logits) at M = 64 193 -> 178 us, 160 292 -> 188, 257 414 -> 265, 512 570 ->
+// 390; 4096 x 6144 x 2560 181 -> 119; M = 45 at 4256 x 1408 21.8 -> 11.0; over
+// 51 shapes (M 33 .. 4096) 0.50 to 0.996 of its time, 0.70 in the mean.
+//
+// The register-staged kernel, for larger operands:
 //   * 128 x 128 output tile per 256-thread workgroup, 2 x 2 waves of
 //     64 x 64, each wave 4 x 4 v_mfma_f32_16x16x32_bf16 per 32-wide K step,
 //     two steps per 64-element (128-byte) chunk; the MFMAs accumulate in
@@ -20,7 +34,10 @@
 //   * epilogue: the residual (the output buffer's bf16 or f32 values) is
 //     added in f32 before the one rounding; rows past M and columns past N
 //     are computed on clamped rows and not stored.
-#include "heph_kernels.h"
+#include <algorithm>
+
+#include "gemm_big.h"
+#include "gemm_ring.h"
 
 namespace heph {
 
@@ -146,10 +163,86 @@ __global__ __launch_bounds__(256, 2) void bf16_gemm_kernel(Bf16GemmArgs a)
     }
 }
 
+namespace {
+
+// Tiles of the DMA-staged kernels and the model that picks one: with n tiles
+// on the fullest CU and KC chunks of 64 elements, n g + KC max(c1, n c) + 2 us,
+// but at least the weights and the output at 5 TB/s, the rate the tiles reach
+// where the stream bounds them; ties go to the earlier entry. c1 is a chunk's
+// latency with one workgroup on the CU, c its share of the CU, g a tile's
+// prologue and epilogue; fitted to MI355X times at 51 shapes (M 33 .. 4096,
+// N 4096 .. 151936, K 1024 .. 2560), over which the choice is on average 3 %
+// slower than the fastest tile.
+struct Bf16Tile {
+    int bm, bn;
+    double g, c1, c;
+    const char* name;
+};
+enum { kT160x320, kT160x256, kT128x256, kT256x256, kT288x192, kT128x128, kT64x64 };
+constexpr Bf16Tile kBf16Tiles[] = {
+    {160, 320, 4.08, 0.109, 1.341, "bf16_gemm_160x320"},
+    {160, 256, 3.53, 1.003, 1.159, "bf16_gemm_160x256"},
+    {128, 256, 3.46, 0.299, 1.047, "bf16_gemm_128x256"},
+    {256, 256, 4.00, 1.005, 1.334, "bf16_gemm_256x256"},
+    {288, 192, 4.00, 1.004, 1.156, "bf16_gemm_288x192"},
+    {128, 128, 1.92, 0.500, 0.699, "bf16_gemm_128x128"},
+    {64, 64, 0.34, 0.410, 0.300, "bf16_gemm_64x64"},
+};
+
+}  // namespace
+
+// The 128- to 288-row tiles of gemm_big.h from M = 65 on (up to 64 rows they
+// would be at most half full); outputs narrower than 4096 columns, where the
+// fit has no shapes, keep the 128 x 128 tile.
+int bf16_gemm_tile(int M, int N, int K, bool c_f32)
+{
+    const double floor_us =
+        3.0 + (2.0 * N * K + (double)M * N * (c_f32 ? 4 : 2)) / 5.0e6;
+    int best = kT128x128;
+    double best_t = -1.0;
+    for (int i = 0; i <= kT64x64; ++i) {
+        const Bf16Tile& t = kBf16Tiles[i];
+        if (N < 4096 && i != kT128x128) continue;
+        if (M <= 64 && i < kT128x128) continue;
+        const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        const double n = (double)((tiles + kPlanCUs - 1) / kPlanCUs), kc = K / 64;
+        const double us = std::max(floor_us, 2.0 + n * t.g + kc * std::max(t.c1, n * t.c));
+        if (best_t < 0.0 || us < best_t) {
+            best_t = us;
+            best = i;
+        }
+    }
+    return best;
+}
+
 hipError_t launch_bf16_gemm(void* c, bool c_f32, bool residual, const uint16_t* x,
                             const uint16_t* w, int M, int N, int K, hipStream_t stream,
                             const LaunchTiming& t, const char** name)
 {
+    if ((long)M * K < (1L << 30) && (long)N * K < (1L << 30)) {
+        Fp8Operands op{};
+        op.x = x;
+        op.w = reinterpret_cast<const uint8_t*>(w);
+        op.c = c;
+        op.c_f32 = c_f32;
+        op.residual = residual;
+        op.M = M;
+        op.N = N;
+        op.K = K;
+        const int i = bf16_gemm_tile(M, N, K, c_f32);
+        const Bf16Tile& b = kBf16Tiles[i];
+        const dim3 grid(((M + b.bm - 1) / b.bm) * ((N + b.bn - 1) / b.bn));
+        *name = b.name;
+        switch (i) {
+        case kT160x320: return launch(fp8_gemm256_kernel<kBigBf16, 160, 320>, grid, dim3(512), 0, stream, t, op);
+        case kT160x256: return launch(fp8_gemm256_kernel<kBigBf16, 160, 256>, grid, dim3(512), 0, stream, t, op);
+        case kT128x256: return launch(fp8_gemm256_kernel<kBigBf16, 128, 256>, grid, dim3(512), 0, stream, t, op);
+        case kT256x256: return launch(fp8_gemm256_kernel<kBigBf16, 256, 256>, grid, dim3(512), 0, stream, t, op);
+        case kT288x192: return launch(fp8_gemm256_kernel<kBigBf16, 288, 192>, grid, dim3(512), 0, stream, t, op);
+        case kT128x128: return launch(gemm_ring_kernel<kRingBf16, 128, 128, 2, 4>, grid, dim3(256), 0, stream, t, op);
+        default: return launch(gemm_ring_kernel<kRingBf16, 64, 64, 2, 4>, grid, dim3(256), 0, stream, t, op);
+        }
+    }
     const Bf16GemmArgs a{c, x, w, M, N, K, c_f32, residual};
     const long tiles = (long)((M + kGbM - 1) / kGbM) * ((N + kGbN - 1) / kGbN);
     if (tiles > 0x7fffffffL) return hipErrorInvalidValue;

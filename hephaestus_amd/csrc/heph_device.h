@@ -42,6 +42,17 @@ __device__ __forceinline__ f32x4 mfma_bf16(const bf16x8& a, const bf16x8& b,
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// D = A(16x64, bf16) * B(64x16, bf16) + C from two 16-byte pieces a lane:
+// the first holds K positions s*8 .. +7 (s = lane >> 4) of the first 32, the
+// second those of the other 32.
+__device__ __forceinline__ f32x4 mfma_bf16x64(const i32x8& a, const i32x8& b, const f32x4& c)
+{
+    const f32x4 d = mfma_bf16(__builtin_bit_cast(bf16x8, i32x4{a[0], a[1], a[2], a[3]}),
+                              __builtin_bit_cast(bf16x8, i32x4{b[0], b[1], b[2], b[3]}), c);
+    return mfma_bf16(__builtin_bit_cast(bf16x8, i32x4{a[4], a[5], a[6], a[7]}),
+                     __builtin_bit_cast(bf16x8, i32x4{b[4], b[5], b[6], b[7]}), d);
+}
+
 __device__ __forceinline__ i32x8 join(const i32x4& lo, const i32x4& hi)
 {
     return i32x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};

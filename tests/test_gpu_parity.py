@@ -692,6 +692,39 @@ def test_bf16_gemm(M, N, K, out, resid):
         assert bad.size == 0, (bad.size, bad[:5])
 
 
+@pytest.mark.parametrize("M,N,K,tile", [
+    (33, 4112, 128, "64x64"), (129, 4304, 384, "64x64"), (34, 4240, 640, "64x64"),
+    (65, 24848, 128, "128x128"), (33, 29744, 640, "128x128"), (65, 40976, 128, "128x256"),
+    (65, 32816, 640, "128x256"), (129, 33008, 128, "160x256"), (130, 32880, 384, "160x256"),
+    (226, 40752, 128, "160x320"), (289, 32784, 384, "160x320"), (161, 32880, 384, "288x192"),
+    (321, 27248, 128, "256x256"), (321, 24656, 384, "256x256")])
+@pytest.mark.parametrize("out,resid", [("f32", False), ("bf16", True)])
+def test_bf16_gemm_every_tile(M, N, K, tile, out, resid):
+    # Every DMA-staged tile of the bf16 GEMM where it can go wrong: two chunks
+    # (fewer than the ring's stages), odd multiples, ragged last row and
+    # column tiles (whole 8-row DMA blocks and 16-row MFMA tiles past M), in
+    # both output types. Bounds as test_bf16_gemm: f32 sums of K products
+    # within 1e-5 of the largest result, bf16 within its rounding.
+    x = O.gen_act_bf16(60 + M, M, K)
+    w = bf16_of(O.gen_normal(61 + N, N * K, 0.0, 0.02)).reshape(N, K)
+    ref = O.bf16_linear(x, w)
+    dt = torch.float32 if out == "f32" else torch.bfloat16
+    res = bf16_of(O.gen_normal(63 + M, M * N, 0.0, 1.0)).reshape(M, N)
+    c = dev(res) if resid else torch.zeros(M, N, dtype=dt, device="cuda")
+    HK.linear(c, dev(x), dev(w), M, N, K, add_residual=resid)
+    torch.cuda.synchronize()
+    assert HK.last_kernel() == "bf16_gemm_" + tile, HK.last_kernel()
+    want = ref + (f32_of_bf16(res).astype(np.float64) if resid else 0.0)
+    if out == "f32":
+        got = c.cpu().numpy()
+        assert max_abs_rel(got, want) < 1e-5, max_abs_rel(got, want)
+    else:
+        got = f32_of_bf16(host_bf16(c)).astype(np.float64)
+        bound = 2.0 ** -8 * np.abs(want) + 1e-5 * np.abs(want).max()
+        bad = np.flatnonzero(np.abs(got - want) > bound)
+        assert bad.size == 0, (bad.size, bad[:5])
+
+
 def test_bf16_gemm_lm_head_rows():
     # The lm_head (151936 x 2560) over 64 positions: 8 sampled rows against
     # the oracle (rows of C are independent), greedy argmax agreeing.
