@@ -38,11 +38,13 @@ def _ptr(t: torch.Tensor) -> int:
 
 
 def _call(name: str, *args) -> None:
-    HK._check(getattr(L.lib(), name)(*args), name)
+    status = getattr(L.lib(), name)(*args)
+    if status != L.HEPH_OK:
+        HK._check(status, name)
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return HK._stream(None)
 
 
 # ------------------------------------------------------------- the ops ----

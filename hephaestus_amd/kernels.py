@@ -45,8 +45,15 @@ def _check(status: int, where: str) -> None:
         raise HephError(status, where)
 
 
+# The current stream's handle without the torch.cuda.Stream object around it
+# (0.3 against 2.7 us on the MI355X host; a whole M = 1 linear is ~5 us of GPU).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(ctx) -> int:
     if ctx is None:
+        if _raw_stream is not None:
+            return _raw_stream(torch.cuda.current_device())
         return torch.cuda.current_stream().cuda_stream
     if isinstance(ctx, torch.cuda.Stream):
         return ctx.cuda_stream
@@ -54,6 +61,8 @@ def _stream(ctx) -> int:
 
 
 def _dev(t: torch.Tensor, name: str, dtypes) -> int:
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype in dtypes and t.is_contiguous():
+        return t.data_ptr()
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch tensor")
     if t.device.type != "cuda":
@@ -65,16 +74,19 @@ def _dev(t: torch.Tensor, name: str, dtypes) -> int:
     return t.data_ptr()
 
 
+_BF16, _F32 = (torch.bfloat16,), (torch.float32,)
 _FP8 = (torch.uint8, torch.float8_e4m3fn)
+_OUT_DTYPES = (torch.bfloat16, torch.float32)
 _OUT = {torch.bfloat16: L.HEPH_DTYPE_BF16, torch.float32: L.HEPH_DTYPE_F32}
 
 
 def _weight_block(scale: torch.Tensor, n: int, k: int) -> tuple[int, int]:
     """(w_block_n, w_block_k) implied by the scale tensor's shape."""
-    if scale.numel() == n and (scale.dim() == 1 or (scale.dim() == 2 and scale.shape[1] == 1)):
+    shape = tuple(scale.shape)
+    if shape == (n, 1) or shape == (n,):
         return 1, k
     nb, kb = -(-n // 128), -(-k // 128)
-    if scale.dim() == 2 and tuple(scale.shape) == (nb, kb):
+    if shape == (nb, kb):
         return 128, 128
     raise ValueError(f"scale shape {tuple(scale.shape)} is neither [{n},1] nor [{nb},{kb}]")
 
@@ -86,8 +98,8 @@ def quantize_act_rows_fp8(a_fp8, act_scale, x, m, k, ctx=None, *, group_k=128):
     if a_fp8.numel() < m * k or act_scale.numel() < m * (k // max(group_k, 1)):
         raise HephError(L.HEPH_ERR_WORKSPACE, "quantize_act_rows_fp8")
     s = L.lib().heph_fp8_quant_act(
-        _dev(x, "x", (torch.bfloat16,)), _dev(a_fp8, "a_fp8", _FP8),
-        _dev(act_scale, "act_scale", (torch.float32,)), m, k, group_k, _stream(ctx))
+        _dev(x, "x", _BF16), _dev(a_fp8, "a_fp8", _FP8),
+        _dev(act_scale, "act_scale", _F32), m, k, group_k, _stream(ctx))
     _check(s, "quantize_act_rows_fp8")
 
 
@@ -107,8 +119,8 @@ def rmsnorm_quant_fp8(a_fp8, act_scale, x, gamma, m, k, eps=1e-6, ctx=None, *, g
     if a_fp8.numel() < m * k or act_scale.numel() < m * (k // max(group_k, 1)):
         raise HephError(L.HEPH_ERR_WORKSPACE, "rmsnorm_quant_fp8")
     s = L.lib().heph_rmsnorm_quant_fp8(
-        _dev(a_fp8, "a_fp8", _FP8), _dev(act_scale, "act_scale", (torch.float32,)),
-        _dev(x, "x", (torch.bfloat16,)), _dev(gamma, "gamma", (torch.bfloat16,)), m, k,
+        _dev(a_fp8, "a_fp8", _FP8), _dev(act_scale, "act_scale", _F32),
+        _dev(x, "x", _BF16), _dev(gamma, "gamma", _BF16), m, k,
         float(eps), group_k, _stream(ctx))
     _check(s, "rmsnorm_quant_fp8")
 
@@ -122,7 +134,7 @@ def silu_mul_quant_fp8(a_fp8, act_scale, gate, up, m, n, ld=None, ctx=None, *, g
     if a_fp8.numel() < m * n or act_scale.numel() < m * (n // max(group_k, 1)):
         raise HephError(L.HEPH_ERR_WORKSPACE, "silu_mul_quant_fp8")
     s = L.lib().heph_silu_mul_quant_fp8(
-        _dev(a_fp8, "a_fp8", _FP8), _dev(act_scale, "act_scale", (torch.float32,)),
+        _dev(a_fp8, "a_fp8", _FP8), _dev(act_scale, "act_scale", _F32),
         gate.data_ptr(), up.data_ptr(), m, n, ld, group_k, _stream(ctx))
     _check(s, "silu_mul_quant_fp8")
 
@@ -151,11 +163,11 @@ def _linear_fp8(c, a, w, scale, a_fp8_ws, act_scale_ws, m, n, k, ctx, *,
         f |= L.FLAG_ADD_RESIDUAL
     if not do_quantize:
         f |= L.FLAG_SKIP_QUANT
-    x_ptr = _dev(a, "a", (torch.bfloat16,)) if do_quantize else (a.data_ptr() if a is not None else None)
-    args = (_dev(c, "c", tuple(_OUT)), _OUT[c.dtype], x_ptr,
-            _dev(w, "w", _FP8), _dev(scale, "scale", (torch.float32,)), bn, bk,
+    x_ptr = _dev(a, "a", _BF16) if do_quantize else (a.data_ptr() if a is not None else None)
+    args = (_dev(c, "c", _OUT_DTYPES), _OUT[c.dtype], x_ptr,
+            _dev(w, "w", _FP8), _dev(scale, "scale", _F32), bn, bk,
             _dev(a_fp8_ws, "a_fp8_ws", _FP8), a_fp8_ws.numel(),
-            _dev(act_scale_ws, "act_scale_ws", (torch.float32,)), act_scale_ws.numel(),
+            _dev(act_scale_ws, "act_scale_ws", _F32), act_scale_ws.numel(),
             m, n, k, group_k, f, _stream(ctx))
     if tune:
         s = L.lib().heph_fp8_linear_with(*args, ctypes.byref(_overrides(tune)))
@@ -176,11 +188,11 @@ def linear_fp8_rmsnorm(c, x, gamma, eps, w, scale, a_fp8_ws, act_scale_ws, n, k,
     if c.numel() < n or w.numel() < n * k or x.numel() < k or gamma.numel() < k:
         raise HephError(L.HEPH_ERR_SHAPE, "linear_fp8_rmsnorm")
     s = L.lib().heph_fp8_linear_rmsnorm(
-        _dev(c, "c", tuple(_OUT)), _OUT[c.dtype], _dev(x, "x", (torch.bfloat16,)),
-        _dev(gamma, "gamma", (torch.bfloat16,)), float(eps),
-        _dev(w, "w", _FP8), _dev(scale, "scale", (torch.float32,)), bn, bk,
+        _dev(c, "c", _OUT_DTYPES), _OUT[c.dtype], _dev(x, "x", _BF16),
+        _dev(gamma, "gamma", _BF16), float(eps),
+        _dev(w, "w", _FP8), _dev(scale, "scale", _F32), bn, bk,
         _dev(a_fp8_ws, "a_fp8_ws", _FP8), a_fp8_ws.numel(),
-        _dev(act_scale_ws, "act_scale_ws", (torch.float32,)), act_scale_ws.numel(),
+        _dev(act_scale_ws, "act_scale_ws", _F32), act_scale_ws.numel(),
         n, k, L.FLAG_ADD_RESIDUAL if add_residual else 0, _stream(ctx))
     _check(s, "linear_fp8_rmsnorm")
 
@@ -212,12 +224,12 @@ def linear_fp8_swiglu(act, x, gamma, eps, w, scale, a_fp8_ws, act_scale_ws, n, k
     if act.numel() < n // 2 or w.numel() < n * k or x.numel() < k or \
             (gamma is not None and gamma.numel() < k):
         raise HephError(L.HEPH_ERR_SHAPE, "linear_fp8_swiglu")
-    g = _dev(gamma, "gamma", (torch.bfloat16,)) if gamma is not None else None
+    g = _dev(gamma, "gamma", _BF16) if gamma is not None else None
     s = L.lib().heph_fp8_linear_swiglu(
-        _dev(act, "act", (torch.bfloat16,)), _dev(x, "x", (torch.bfloat16,)), g, float(eps),
-        _dev(w, "w", _FP8), _dev(scale, "scale", (torch.float32,)), bn, bk,
+        _dev(act, "act", _BF16), _dev(x, "x", _BF16), g, float(eps),
+        _dev(w, "w", _FP8), _dev(scale, "scale", _F32), bn, bk,
         _dev(a_fp8_ws, "a_fp8_ws", _FP8), a_fp8_ws.numel(),
-        _dev(act_scale_ws, "act_scale_ws", (torch.float32,)), act_scale_ws.numel(),
+        _dev(act_scale_ws, "act_scale_ws", _F32), act_scale_ws.numel(),
         n, k, _stream(ctx))
     _check(s, "linear_fp8_swiglu")
 
@@ -258,8 +270,8 @@ def linear(c, a, b, m, n, k, ctx=None, *, add_residual=False):
     if c.numel() < m * n or a.numel() < m * k or b.numel() < n * k:
         raise HephError(L.HEPH_ERR_SHAPE, "linear")
     s = L.lib().heph_bf16_linear(
-        _dev(c, "c", tuple(_OUT)), _OUT[c.dtype], _dev(a, "a", (torch.bfloat16,)),
-        _dev(b, "b", (torch.bfloat16,)), m, n, k,
+        _dev(c, "c", _OUT_DTYPES), _OUT[c.dtype], _dev(a, "a", _BF16),
+        _dev(b, "b", _BF16), m, n, k,
         L.FLAG_ADD_RESIDUAL if add_residual else 0, _stream(ctx))
     _check(s, "linear")
 
