@@ -31,6 +31,11 @@ CFLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-munsafe-fp-atomics",
 ]
+# The 256-thread GEMM tiles hold one workgroup of 4 waves on a CU, so the
+# compiler sees 512 registers a lane and puts the MFMA results into the
+# accumulation half, copying them at every loop end; this keeps them in
+# ordinary registers (no copies, 10 % less time at 128 x 64).
+FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("gemm.hip", "bf16_gemm.hip")}
 
 
 def sources():
@@ -39,7 +44,7 @@ def sources():
 
 def _compile(src: str) -> str:
     obj = os.path.join(BUILD, os.path.basename(src)[:-4] + ".o")
-    cmd = [HIPCC, *CFLAGS, "-c", src, "-o", obj]
+    cmd = [HIPCC, *CFLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed on {src}:\n{r.stdout}\n{r.stderr}")

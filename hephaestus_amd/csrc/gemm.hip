@@ -26,6 +26,7 @@
 #include <algorithm>
 
 #include "gemm_big.h"
+#include "gemm_ring.h"
 
 namespace heph {
 
@@ -197,8 +198,11 @@ __global__ __launch_bounds__(256, 2) void fp8_gemm_kernel(Fp8Operands op)
         }
 }
 
-// Sums the K-split partials of the large-M GEMM in split order, adds the
-// residual and stores bf16 or f32 (four outputs per thread; N % 16 == 0).
+// Sums the K-split partials of a GEMM in split order, applies per-token and
+// per-channel scales where nothing varied along K ((acc*sa)*sw, the
+// association of the unsplit tiles), adds the residual and stores bf16 or f32
+// (four outputs per thread; N % 16 == 0).
+template <bool SCALE>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(Fp8Operands op)
 {
     const size_t mn = (size_t)op.M * op.N, n4 = mn / 4;
@@ -207,6 +211,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(Fp8Operands op)
          i += (size_t)gridDim.x * 256) {
         f32x4 v = part[i];
         for (int s = 1; s < op.splits; ++s) v += part[(size_t)s * n4 + i];
+        if constexpr (SCALE) {
+            const size_t row = i * 4 / op.N;
+            const float sa = op.s[row];
+            const f32x4 sw = *reinterpret_cast<const f32x4*>(op.sw + (i * 4 - row * op.N));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (v[e] * sa) * sw[e];
+        }
         if (op.c_f32) {
             f32x4* c = static_cast<f32x4*>(op.c) + i;
             if (op.residual) v += *c;
@@ -229,7 +240,9 @@ hipError_t launch_splitk_reduce(const Fp8Operands& op, hipStream_t stream, const
 {
     const size_t n4 = (size_t)op.M * op.N / 4;
     const int blocks = (int)std::min<size_t>((n4 + 255) / 256, 4096);
-    return launch(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, stream, t, op);
+    if (op.s_step == 0)
+        return launch(splitk_reduce_kernel<true>, dim3(blocks), dim3(256), 0, stream, t, op);
+    return launch(splitk_reduce_kernel<false>, dim3(blocks), dim3(256), 0, stream, t, op);
 }
 
 namespace {
@@ -256,6 +269,26 @@ hipError_t launch_big(const Fp8Operands& op, hipStream_t stream, const LaunchTim
     if (op.s_step == 0)
         return launch(fp8_gemm256_kernel<2, BM, BN>, grid, dim3(512), 0, stream, t, op);
     return launch(fp8_gemm256_kernel<1, BM, BN>, grid, dim3(512), 0, stream, t, op);
+}
+
+template <int SM, int BM, int BN, int D>
+hipError_t launch_ring_t(const Fp8Operands& op, hipStream_t stream, const LaunchTiming& t)
+{
+    const dim3 grid(((op.M + BM - 1) / BM) * ((op.N + BN - 1) / BN) * op.splits);
+    if (op.splits == 1)
+        return launch(gemm_ring_kernel<SM, BM, BN, 2, D>, grid, dim3(256), 0, stream, t, op);
+    hipError_t e = launch(gemm_ring_kernel<SM, BM, BN, 2, D>, grid, dim3(256), 0, stream,
+                          LaunchTiming{t.start, nullptr}, op);
+    if (e != hipSuccess) return e;
+    return launch_splitk_reduce(op, stream, LaunchTiming{nullptr, t.stop});
+}
+
+template <int BM, int BN, int D>
+hipError_t launch_ring(const Fp8Operands& op, hipStream_t stream, const LaunchTiming& t)
+{
+    if (op.w_block) return launch_ring_t<kRingBlock, BM, BN, D>(op, stream, t);
+    if (op.s_step == 0) return launch_ring_t<kRingConst, BM, BN, D>(op, stream, t);
+    return launch_ring_t<kRingChannel, BM, BN, D>(op, stream, t);
 }
 
 }  // namespace
@@ -298,18 +331,53 @@ static double gemm_estimate(int M, int N, int K, const TileCost& tc, int s, long
     return t;
 }
 
+// The ring tiles (gemm_ring.h) and their cost: with n workgroups on the fullest
+// CU, KC chunks each and weights streamed at 5 TB/s at best,
+//     max(2 + n g + KC max(c1, n c), 3 + N K / 5e6) us,
+// a split's reduction 2.5 us and its partials at 4 TB/s (c1 a chunk's latency
+// alone on the CU, c its share of it; fitted to 1230 MI355X times at 47 shapes,
+// M 33 .. 1000, N 1024 .. 19456, K 1024 .. 9728, 1 .. 8 splits, weights from
+// HBM).
+struct RingCost {
+    int bm, bn;
+    double g, c1, c;
+};
+constexpr RingCost kRingCost[] = {{64, 64, 1.42, 0.310, 0.274},
+                                  {64, 32, 0.65, 0.276, 0.213},
+                                  {96, 64, 2.74, 0.242, 0.357},
+                                  {64, 128, 3.41, 0.319, 0.424}};
+
+static double ring_estimate(int M, int N, int K, const RingCost& rc, int s)
+{
+    const long wgs = (long)((M + rc.bm - 1) / rc.bm) * ((N + rc.bn - 1) / rc.bn) * s;
+    const double n = (double)((wgs + kPlanCUs - 1) / kPlanCUs);
+    const int kc = (K / kChunk + s - 1) / s;
+    const double t = std::max(2.0 + n * rc.g + kc * std::max(rc.c1, n * rc.c),
+                              3.0 + (double)N * K / 5.0e6);
+    return s > 1 ? t + 2.5 + (double)s * M * N * 4.0 / 4.0e6 : t;
+}
+
 // Tile and K splits of the large-M GEMM: the pair with the least estimated
 // time, splitting only when allowed, into at most 8 splits of at least 4
 // chunks; ties go to the earlier tile of kTileCost, then to fewer splits.
 // A forced tile height (gemm_bm) or width (gemm_bn) keeps only the tiles
-// that have it.
-GemmPlan gemm_plan(int M, int N, int K, bool can_split, int forced_bm, int forced_bn)
+// that have it. per_token (nothing varies along K): the large tiles do not
+// split.
+// From 33 to 511 rows (per-token scales: to 1023, where the alternative is a
+// large tile over all of K) a ring tile is taken where its estimate is under 0.8 of
+// that: over the 47 shapes of its fit the choice then ran at 0.80 (block
+// scales) and 0.69 (per-token) of the large tiles' time, 1.02 at worst (0.8 to
+// 1.0: up to 1.19; from M = 470 on the two run alike). Past K = 4096 the ring
+// always splits where it may: one workgroup's chain of chunks is then longer
+// than a reduction.
+GemmPlan gemm_plan(int M, int N, int K, bool can_split, int forced_bm, int forced_bn,
+                   bool per_token)
 {
     // MI355X's 256 CUs, not the visible count: the plan (and the K-split
     // summation order with it) does not change under a CU mask or partition
     const long cus = kPlanCUs;
     const int KC = K / kChunk;
-    GemmPlan best{0, 0, 1};
+    GemmPlan best{0, 0, 1, false};
     double best_t = -1.0;
     for (const auto& tc : kTileCost) {
         // 64 x 192 only where its fit holds (M >= 256): below, the K-split
@@ -317,23 +385,36 @@ GemmPlan gemm_plan(int M, int N, int K, bool can_split, int forced_bm, int force
         if (tc.bm == 64 && tc.bn == 192 && M < 256 && forced_bn != 192) continue;
         if (forced_bm >= 64 && tc.bm != forced_bm) continue;
         if (forced_bn && tc.bn != forced_bn) continue;
-        for (int s = 1; s <= (can_split ? 8 : 1); ++s) {
+        for (int s = 1; s <= (can_split && !per_token ? 8 : 1); ++s) {
             if (s > 1 && KC / s < 4) break;
             const double t = gemm_estimate(M, N, K, tc, s, cus);
             if (best_t < 0.0 || t < best_t) {
                 best_t = t;
-                best = GemmPlan{tc.bm, tc.bn, s};
+                best = GemmPlan{tc.bm, tc.bn, s, false};
             }
         }
     }
-    if (best.bm == 0) best = GemmPlan{forced_bm >= 64 ? forced_bm : 256, 256, 1};
+    if (best.bm == 0) best = GemmPlan{forced_bm >= 64 ? forced_bm : 256, 256, 1, false};
+    if (M <= 32 || M >= (per_token ? 1024 : 512) || forced_bm || forced_bn) return best;
+    best_t *= 0.8;
+    for (const auto& rc : kRingCost) {
+        for (int s = can_split && K > 4096 ? 2 : 1; s <= (can_split ? 8 : 1); ++s) {
+            if (s > 1 && KC / s < 4) break;
+            const double t = ring_estimate(M, N, K, rc, s);
+            if (t < best_t) {
+                best_t = t;
+                best = GemmPlan{rc.bm, rc.bn, s, true};
+            }
+        }
+    }
     return best;
 }
 
 bool gemm_splits_ready(const Fp8Operands& op)
 {
-    if (!op.part || op.s_step == 0) return false;
-    const int s = gemm_plan(op.M, op.N, op.K, true, op.tune.gemm_bm, op.tune.gemm_bn).splits;
+    if (!op.part) return false;
+    const int s = gemm_plan(op.M, op.N, op.K, true, op.tune.gemm_bm, op.tune.gemm_bn,
+                            op.s_step == 0).splits;
     return s > 1 && op.part_bytes >= (size_t)s * op.M * op.N * 4;
 }
 
@@ -354,13 +435,28 @@ hipError_t launch_fp8_gemm(const Fp8Operands& op, hipStream_t stream,
     const bool small_offsets = (long)op.M * op.K < (1L << 31) && (long)op.N * op.K < (1L << 31);
     const bool force_128 = op.tune.gemm_bm == 1;
     if (small_offsets && !force_128) {
-        // K splits when the caller's scratch holds their partials (block or
-        // per-channel weights with per-chunk activation scales).
+        // K splits when the caller's scratch holds their partials.
         Fp8Operands o = op;
         const GemmPlan plan = gemm_plan(o.M, o.N, o.K, gemm_splits_ready(o), o.tune.gemm_bm,
-                                        o.tune.gemm_bn);
+                                        o.tune.gemm_bn, o.s_step == 0);
         o.splits = plan.splits;
         const bool sk = o.splits > 1;
+        if (plan.ring) {
+            if (plan.bm == 96) {
+                *name = sk ? "fp8_gemm_96x64_splitk" : "fp8_gemm_96x64";
+                return launch_ring<96, 64, 6>(o, stream, t);
+            }
+            if (plan.bn == 64) {
+                *name = sk ? "fp8_gemm_64x64_splitk" : "fp8_gemm_64x64";
+                return launch_ring<64, 64, 4>(o, stream, t);
+            }
+            if (plan.bn == 32) {
+                *name = sk ? "fp8_gemm_64x32_splitk" : "fp8_gemm_64x32";
+                return launch_ring<64, 32, 4>(o, stream, t);
+            }
+            *name = sk ? "fp8_gemm_64x128_splitk" : "fp8_gemm_64x128";
+            return launch_ring<64, 128, 6>(o, stream, t);
+        }
         if (plan.bn == 192 && plan.bm == 64) {
             *name = sk ? "fp8_gemm_64x192_splitk" : "fp8_gemm_64x192";
             return launch_big<64, 192>(o, stream, t);

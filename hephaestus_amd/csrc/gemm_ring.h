@@ -1,9 +1,31 @@
 // gemm_ring.h - GEMM tiles for the sizes between batched decode and long
 // prefill: a 256-thread workgroup per BM x BN output tile, operands through
-// a D-stage LDS ring filled by DMA (included by gemm_ring.hip).
+// a D-stage LDS ring filled by DMA (included by gemm.hip and bf16_gemm.hip).
+//
+// At these sizes (M of 33 to a few hundred) the 512-thread tiles of gemm_big.h
+// leave most CUs idle, so tiles are small, and a small tile's chunk is short:
+// what bounds it is whatever the wave does one after the other. On MI355X a
+// 128 x 64 E4M3 chunk costs ~400 cycles of DMA (24 KB into LDS at ~60 B a
+// cycle and CU, the L2's rate), 256 of MFMA and ~200 of LDS reads; with the
+// chunk's fragments read after its barrier the four waves, in step, paid the
+// sum (950 cycles). Hence:
+//   * a chunk's fragments are read into registers while the chunk before it is
+//     contracted (two sets), and the ring's refill goes out between the row
+//     tiles' MFMAs: 456 cycles a chunk;
+//   * the steady loop has no branch. The compiler waits for every LDS read in
+//     flight (lgkmcnt(0)) at a join of control flow, which serialized the
+//     same steps again (tiles inside M, ragged tiles and waves without rows
+//     are separate copies of the loop);
+//   * no scalar load is in flight beside LDS reads, for the same reason;
+//   * the stages are a few more than the DMA's latency needs: two workgroups
+//     of 64 KB, or one of up to 150 KB, share a CU.
+// M = 333, 4096 x 2560 per-channel: 12.8 -> 9.8 us; M = 48, 2560 x 9728 block
+// scales: 18.6 -> 13.9 with its reduction (kernel times, graph-replayed over
+// HBM-streamed weights; before: gemm_big.h's 64 x 192 and 64 x 256 x 8 splits).
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "gemm_dma.h"
 
@@ -11,6 +33,7 @@ namespace heph {
 
 namespace {
 
+// What the tile contracts, as BigType in gemm_big.h.
 enum RingType { kRingBlock = 0, kRingChannel = 1, kRingConst = 2, kRingBf16 = 3 };
 
 // s_waitcnt: at most N vector memory instructions and no LDS or scalar one
@@ -52,11 +75,10 @@ struct RingTile {
     static_assert(128 % WN == 0 || SM >= 2, "a wave's columns lie in one weight block");
     static_assert(!SCALES || SROWS <= 4, "a wave moves the scales of 64 rows");
     static_assert(D >= 2 && BYTES <= 160 * 1024, "LDS");
-    static constexpr int WGS = BYTES * 2 <= 160 * 1024 ? 2 : 1;    // workgroups per CU
 };
 
 template <int SM, int BM, int BN, int WGM, int D>
-__global__ __launch_bounds__(256, (RingTile<SM, BM, BN, WGM, D>::WGS)) void gemm_ring_kernel(
+__global__ __launch_bounds__(256, 2) void gemm_ring_kernel(
     Fp8Operands op)
 {
     using T = RingTile<SM, BM, BN, WGM, D>;
@@ -98,19 +120,18 @@ __global__ __launch_bounds__(256, (RingTile<SM, BM, BN, WGM, D>::WGS)) void gemm
     const int sp = wave % T::SROWS;
     const uint32_t soff = (uint32_t)min(m0 + sp * 64 + lane, M - 1) * (uint32_t)op.s_ld * 4u;
     const uint32_t s_step = (uint32_t)op.s_step * 4u;
-    const bool full = m0 + BM <= M;              // no block of A left out
-    const bool live = m0 + wm * T::WM < M;       // this wave has rows to contract
-    auto issue = [&](int j, int st) {
+    // DMA instruction `part` of stage st: A's blocks, the row scales, B's blocks
+    auto issue_part = [&](auto fullc, int j, int st, int part) {
         uint8_t* base = smem + st * T::STAGE;
-#pragma unroll
-        for (int q = 0; q < T::NA; ++q)
-            if (full || m0 + (q * 4 + wave) * 8 < M)
-                dma16(rq, aoff[q], (uint32_t)j * kChunk, base + (q * 4 + wave) * 1024);
-        if constexpr (T::SCALES)
+        if (part < T::NA) {
+            if (decltype(fullc)::value || m0 + (part * 4 + wave) * 8 < M)
+                dma16(rq, aoff[part], (uint32_t)j * kChunk, base + (part * 4 + wave) * 1024);
+        } else if (T::SCALES && part == T::NA) {
             dma4(rs, soff, (uint32_t)j * s_step, base + T::A + T::B + sp * 256);
-#pragma unroll
-        for (int q = 0; q < T::NB; ++q)
+        } else {
+            const int q = part - (T::P - T::NB);
             dma16(rw, boff[q], (uint32_t)j * kChunk, base + T::A + (q * 4 + wave) * 1024);
+        }
     };
 
     float swc[NT][4];
@@ -137,34 +158,60 @@ __global__ __launch_bounds__(256, (RingTile<SM, BM, BN, WGM, D>::WGS)) void gemm
 #pragma unroll
         for (int ni = 0; ni < NT; ++ni) acc[mi][ni] = f32x4{0, 0, 0, 0};
 
+    // The fragments of a chunk in registers: read while the MFMAs of the
+    // chunk before it run.
+    struct Frags {
+        i32x8 a[MT], b[NT];
+        float sa[MT];
+    };
+    auto read_a = [&](Frags& f, int st, int mi) {
+        const uint8_t* p = smem + st * T::STAGE + a_row + mi * 16 * kChunk;
+        f.a[mi] = join(*reinterpret_cast<const i32x4*>(p + sl0),
+                       *reinterpret_cast<const i32x4*>(p + sl1));
+        if constexpr (T::SCALES)
+            f.sa[mi] = *reinterpret_cast<const float*>(smem + st * T::STAGE + s_row + mi * 64);
+    };
+    auto read_b = [&](Frags& f, int st, int ni) {
+        const uint8_t* p = smem + st * T::STAGE + b_row + ni * 16 * kChunk;
+        f.b[ni] = join(*reinterpret_cast<const i32x4*>(p + sl0),
+                       *reinterpret_cast<const i32x4*>(p + sl1));
+    };
+    // All of K for one tile. FULL: every row block of A is inside M; else the
+    // blocks past it are left out, and a stage's wait counts the others only
+    // (the newest). LIVE: this wave has rows to contract. Both are fixed before
+    // the loop, whose steady part (the ring not yet draining) then has no
+    // branch: across one, the compiler waits for every LDS read in flight.
+    auto contract_tile = [&](auto fullc, auto livec) {
+        constexpr bool FULL = decltype(fullc)::value, LIVE = decltype(livec)::value;
+        constexpr int PW = FULL ? T::P : T::NB + (T::SCALES ? 1 : 0);
 #pragma unroll
-    for (int d = 0; d < D - 1; ++d)
-        if (jb + d < je) issue(jb + d, d);
-    float sw_cur = SM == kRingBlock ? swb[jb] : 1.0f, sw_nxt = 1.0f;
-
-    int st = 0;
-    for (int j = jb; j < je; ++j) {
-        // a tile with blocks left out counts the others only (the newest)
-        if (full) wait_ring<T::P, D - 2>(je - 1 - j);
-        else wait_ring<T::NB + (T::SCALES ? 1 : 0), D - 2>(je - 1 - j);
+        for (int d = 0; d < D; ++d)
+            if (jb + d < je)
+#pragma unroll
+                for (int part = 0; part < T::P; ++part) issue_part(fullc, jb + d, d, part);
+        float sw_cur = SM == kRingBlock ? swb[jb] : 1.0f;
+        Frags f0, f1;
+        wait_ring<PW, D - 1>(min(D - 1, je - 1 - jb));
         stage_barrier();
-        const uint8_t* stp = smem + st * T::STAGE;
-        auto frag = [&](int off) {
-            return join(*reinterpret_cast<const i32x4*>(stp + off + sl0),
-                        *reinterpret_cast<const i32x4*>(stp + off + sl1));
-        };
-        i32x8 b[NT], a[2];
-        float sa[2] = {0.0f, 0.0f};
-        if (live) {
+        if constexpr (LIVE) {
 #pragma unroll
-            for (int ni = 0; ni < NT; ++ni) b[ni] = frag(b_row + ni * 16 * kChunk);
-            a[0] = frag(a_row);
-            if constexpr (T::SCALES) sa[0] = *reinterpret_cast<const float*>(stp + s_row);
+            for (int ni = 0; ni < NT; ++ni) read_b(f0, 0, ni);
+#pragma unroll
+            for (int mi = 0; mi < MT; ++mi) read_a(f0, 0, mi);
         }
-        if (j + D - 1 < je) issue(j + D - 1, st == 0 ? D - 1 : st - 1);
-        if constexpr (SM == kRingBlock)
-            if (j + 1 < je) sw_nxt = swb[j + 1];
-        if (live) {
+        // One chunk: wait until the next one is in and every wave has its
+        // fragments of this one (the barrier); then, between the row tiles'
+        // MFMAs, read the next chunk's fragments and refill this one's stage.
+        int st = 0;
+        auto step = [&](auto steadyc, Frags& cur, Frags& nxt, int j) {
+            constexpr bool STEADY = decltype(steadyc)::value;
+            const int sn = st + 1 == D ? 0 : st + 1;
+            const bool more = STEADY || j + 1 < je;
+            if (more) {
+                if constexpr (STEADY) wait_vm<(D - 2) * PW>();
+                else wait_ring<PW, D - 2>(je - 2 - j);
+                stage_barrier();
+            }
             f32x4 p[2][NT];
             float sc[2] = {0.0f, 0.0f};
             auto rescale = [&](int mi) {
@@ -177,31 +224,57 @@ __global__ __launch_bounds__(256, (RingTile<SM, BM, BN, WGM, D>::WGS)) void gemm
             };
 #pragma unroll
             for (int mi = 0; mi < MT; ++mi) {
-                const int cur = mi & 1;
-                if (mi + 1 < MT) {
-                    a[cur ^ 1] = frag(a_row + (mi + 1) * 16 * kChunk);
-                    if constexpr (T::SCALES)
-                        sa[cur ^ 1] = *reinterpret_cast<const float*>(stp + s_row + (mi + 1) * 64);
+                if constexpr (LIVE) {
+                    if (more) {
+#pragma unroll
+                        for (int ni = mi * NT / MT; ni < (mi + 1) * NT / MT; ++ni) read_b(nxt, sn, ni);
+                        read_a(nxt, sn, mi);
+                    }
+                    if constexpr (SM == kRingBf16) {
+#pragma unroll
+                        for (int ni = 0; ni < NT; ++ni)
+                            acc[mi][ni] = mfma_bf16x64(cur.b[ni], cur.a[mi], acc[mi][ni]);
+                    } else if constexpr (SM == kRingConst) {
+#pragma unroll
+                        for (int ni = 0; ni < NT; ++ni)
+                            acc[mi][ni] = mfma_e4m3(cur.b[ni], cur.a[mi], acc[mi][ni]);
+                    } else {
+                        sc[mi & 1] = cur.sa[mi] * sw_cur;
+#pragma unroll
+                        for (int ni = 0; ni < NT; ++ni)
+                            p[mi & 1][ni] = mfma_e4m3(cur.b[ni], cur.a[mi], f32x4{0, 0, 0, 0});
+                        if (mi > 0) rescale(mi - 1);
+                    }
                 }
-                if constexpr (SM == kRingBf16) {
+                if constexpr (STEADY) {
 #pragma unroll
-                    for (int ni = 0; ni < NT; ++ni) acc[mi][ni] = mfma_bf16x64(b[ni], a[cur], acc[mi][ni]);
-                } else if constexpr (SM == kRingConst) {
-#pragma unroll
-                    for (int ni = 0; ni < NT; ++ni) acc[mi][ni] = mfma_e4m3(b[ni], a[cur], acc[mi][ni]);
-                } else {
-                    sc[cur] = sa[cur] * sw_cur;
-#pragma unroll
-                    for (int ni = 0; ni < NT; ++ni)
-                        p[cur][ni] = mfma_e4m3(b[ni], a[cur], f32x4{0, 0, 0, 0});
-                    if (mi > 0) rescale(mi - 1);
+                    for (int part = mi * T::P / MT; part < (mi + 1) * T::P / MT; ++part)
+                        issue_part(fullc, j + D, st, part);
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if constexpr (T::SCALES) rescale(MT - 1);
+            if constexpr (LIVE && T::SCALES) rescale(MT - 1);
+            // after the last LDS read: with a scalar load in flight every wait
+            // for LDS would wait for all of it
+            if constexpr (SM == kRingBlock)
+                if (more) sw_cur = swb[j + 1];
+            st = sn;
+        };
+        int j = jb;
+        for (; j + 1 + D < je; j += 2) {
+            step(std::true_type{}, f0, f1, j);
+            step(std::true_type{}, f1, f0, j + 1);
         }
-        sw_cur = sw_nxt;
-        st = st + 1 == D ? 0 : st + 1;
-    }
+        for (; j + 1 < je; j += 2) {
+            if (j + D < je) step(std::true_type{}, f0, f1, j);
+            else step(std::false_type{}, f0, f1, j);
+            step(std::false_type{}, f1, f0, j + 1);
+        }
+        if (j < je) step(std::false_type{}, f0, f1, j);
+    };
+    if (m0 + BM <= M) contract_tile(std::true_type{}, std::true_type{});
+    else if (m0 + wm * T::WM < M) contract_tile(std::false_type{}, std::true_type{});
+    else contract_tile(std::false_type{}, std::false_type{});
 
     // lane: row r16 and columns 4 slice .. +3 of each 16x16 block
 #pragma unroll
@@ -215,7 +288,7 @@ __global__ __launch_bounds__(256, (RingTile<SM, BM, BN, WGM, D>::WGS)) void gemm
             if (col >= N) continue;
             f32x4 v = acc[mi][ni];
             const size_t o = (size_t)row * N + col;
-            if (SM != kRingConst && S > 1) {
+            if (S > 1) {    // the fp32 partial, unscaled for kRingConst
                 *reinterpret_cast<f32x4*>(op.part + (size_t)split * M * N + o) = v;
                 continue;
             }

@@ -1356,6 +1356,72 @@ def test_large_m_split_k_exact_and_repeatable():
     assert np.array_equal(outs[0], bf16_of(exact.astype(np.float32)))
 
 
+# Shapes that take each ring tile by default, unsplit and split over K: fewer
+# chunks than the ring has stages up to many, row tiles with whole DMA blocks
+# and whole waves past M, ragged columns, ragged splits.
+RING_CASES = [("64x32", 35, 176, 128), ("64x32", 147, 1504, 640), ("64x64", 154, 3952, 256),
+              ("64x64", 67, 4128, 2176), ("96x64", 132, 5456, 896), ("64x128", 196, 5472, 1664),
+              ("64x32_splitk", 39, 144, 4224), ("64x32_splitk", 45, 1776, 2176),
+              ("64x64_splitk", 180, 1424, 4224), ("96x64_splitk", 90, 5408, 4224),
+              ("64x128_splitk", 129, 2800, 4224)]
+
+
+@pytest.mark.parametrize("tile,M,N,K", RING_CASES)
+@pytest.mark.parametrize("mode", ["block", "channel_token", "channel_g128"])
+@pytest.mark.parametrize("out,resid", [("bf16", True), ("f32", False)])
+def test_ring_tiles_vs_oracle(tile, M, N, K, mode, out, resid):
+    x = O.gen_act_bf16(160 + M, M, K, outlier_p=1e-3)
+    if mode == "block":
+        qw, sw = O.gen_weight(161, N, K)
+        bn, bk, g = 128, 128, 128
+    else:
+        qw, sw = O.quant_weight(O.gen_normal(161, N * K, 0.0, 0.02).reshape(N, K), 1, K)
+        bn, bk, g = 1, K, (K if mode == "channel_token" else 128)
+    dt = torch.bfloat16 if out == "bf16" else torch.float32
+    r = O.gen_normal(162, M * N).reshape(M, N).astype(np.float32)
+    res_t = dev(bf16_of(r)) if resid else None
+    q_ws, s_ws = HK.workspace(M, K, group_k=g, n=N)
+    c, q_ws, _ = run_linear(qw, sw, x, M=M, N=N, K=K, group_k=g, out=dt, residual=res_t,
+                            q_ws=q_ws, s_ws=s_ws)
+    assert HK.last_kernel() == "fp8_gemm_" + tile, HK.last_kernel()
+    ref = O.quant_linear(x, qw, sw, group_k=g, bn=bn, bk=bk)
+    if resid:
+        check_close(host_bf16(c), ref + f32_of_bf16(bf16_of(r)), tile)
+    else:
+        got = c.cpu().numpy()
+        assert max_abs_rel(got, ref) <= TOL
+        # the large tile contracts the same chunks in the same order: equal bit
+        # for bit where K is not split, else within the f32 sums' own rounding
+        base, _, _ = run_linear(qw, sw, x, M=M, N=N, K=K, group_k=g, out=dt,
+                                tune={"gemm_bm": 64, "gemm_bn": 256})
+        base = base.cpu().numpy()
+        if tile.endswith("_splitk"):
+            assert max_abs_rel(got, base) <= 1e-6
+        else:
+            assert np.array_equal(got, base)
+    qo, _ = O.quant_act(x, g)
+    assert np.array_equal(q_ws[: M * K].cpu().numpy().reshape(M, K), qo)
+
+
+@pytest.mark.parametrize("tile,M,N,K", RING_CASES)
+def test_ring_tiles_exact_integer(tile, M, N, K):
+    # Every partial sum is an integer below 2^24 times a power of two: bit for
+    # bit, block scales and per-token scales, twice the same.
+    ia, qa = lattice(M, K, 8000 + M)
+    iw, qw = lattice(N, K, 8001)
+    ref = (ia.astype(np.float64) @ iw.astype(np.float64).T) * 0.0625 * 2.0 ** -5
+    for g, sw in ((128, np.full((-(-N // 128), K // 128), 2.0 ** -2, np.float32)),
+                  (K, np.full((N, 1), 2.0 ** -2, np.float32))):
+        q_ws, s_ws = HK.workspace(M, K, group_k=g, n=N)
+        q_ws[: M * K].copy_(dev(qa.reshape(-1)))
+        s_ws.fill_(2.0 ** -3)
+        for _ in range(2):
+            c, _, _ = run_linear(qw, sw, None, M=M, N=N, K=K, group_k=g, skip_quant=True,
+                                 q_ws=q_ws, s_ws=s_ws)
+            assert HK.last_kernel() == "fp8_gemm_" + tile, HK.last_kernel()
+            assert np.array_equal(host_bf16(c), bf16_of(ref.astype(np.float32)))
+
+
 @pytest.mark.parametrize("M", [512, 4096])
 def test_large_m_tile_choice(M):
     # The automatic tile (and K splits, where the workspace holds their
