@@ -16,6 +16,9 @@
 //   * argmax over bf16-rounded logits, lowest index on ties (kernels.mojo:1376-1433)
 // The KV cache holds E4M3 codes with one scale per (layer, kv head, K|V):
 // new rows are quantized as code = e4m3(clamp(v * (1/s), +-448)).
+#include <algorithm>
+#include <type_traits>
+
 #include "heph_kernels.h"
 #include "../../include/hephdecode.h"
 
@@ -255,12 +258,20 @@ __device__ __forceinline__ void decode16(const uint4& w, float* f)
 // Keys per split and per thread of the scores kernel: the split's keys sit
 // in kAttnSplit / kAttnKPT key slots of 8 lanes, a workgroup of
 // 8 * kAttnSplit / kAttnKPT threads; a score's arithmetic does not depend
-// on either. On MI355X at 4097 keys (graph-replayed decode step, ms per
-// token): 256 keys x 2 per thread (136 workgroups of 1024 threads) 1.682,
+// on either. On MI355X at 4097 keys, 4 query heads per kv head (graph-replayed
+// decode step, ms per token): 256 keys x 2 per thread (136 workgroups of 1024 threads) 1.682,
 // 256 x 4 1.687, 128 x 4 1.727, 64 x 2 1.712, 512 x 4 1.743, 256 x 8 1.727:
 // fewer workgroups each prepare the query heads once for more keys.
 constexpr int kAttnSplit = 256;
-constexpr int kAttnKPT = 2;
+// With 8 query heads a thread holds 128 floats of q: at 1024 threads (128
+// registers each) they spilled, so 512 threads take 4 keys each (the attention
+// at 4 kv x 8 query heads: 4097 keys 19.0 -> 13.5 us, 20000 66.1 -> 30.7).
+template <int G>
+constexpr int kAttnKPT = G == 8 ? 4 : 2;
+// Scores workgroups that MI355X holds at once: two 1024-thread ones on each of
+// its 256 CUs with one query head (54 registers), else one.
+template <int G>
+constexpr int kAttnSlots = (G == 1 ? 2 : 1) * kPlanCUs;
 
 // The workspace holds the scores [n_heads][n_keys] (fp32).
 
@@ -311,27 +322,36 @@ struct QkvPrep {
 // q heads and the new key's codes meet in LDS after one barrier, and the
 // new key's score uses those codes instead of the cache row loaded at the
 // start. All of it runs while the cache loads are in flight.
-template <int G, bool QKV, int KPT>
+//
+// LOOP: a workgroup takes every `stride`-th split from its first on, loading the
+// next split's rows before it scores the current one: with more splits than
+// workgroups fit the device (kAttnSlots), each prepares its q heads once and no
+// second round of workgroups starts behind the first (the attention at 8 kv x 4
+// query heads, graph-replayed: 8193 keys 19.7 -> 18.4 us, 40000 59.3 -> 53.8).
+template <int G, bool QKV, int KPT, bool LOOP>
 __global__ __launch_bounds__(8 * kAttnSplit / KPT) void attn_scores_kernel(
     float* ws, const uint16_t* q, const uint8_t* kc, const float* kv_scale, int n_kv,
-    int n_keys, int n_splits, QkvPrep prep)
+    int n_keys, int n_splits, int stride, QkvPrep prep)
 {
     constexpr int D = 128;
     constexpr int SLOTS = kAttnSplit / KPT, NW = SLOTS / 8;   // key slots, waves
-    const int kh = blockIdx.x % n_kv, split = blockIdx.x / n_kv;
+    const int kh = blockIdx.x % n_kv, split0 = blockIdx.x / n_kv;
     const int t = threadIdx.x, ks = t >> 3, c = t & 7;
     const size_t row = (size_t)n_kv * D;
-    const int j0 = split * kAttnSplit + ks;
+    // whether this workgroup scores the split holding the newest key
+    const bool last = LOOP ? (n_splits - 1 - split0) % stride == 0 : split0 == n_splits - 1;
     // The cache rows go out after the loads of q (or of the raw projection
     // row and the norm gammas): a wave's loads complete in issue order, and
     // the q preparation, which needs only those, then runs while the cache
     // rows are in flight.
     uint4 kv[KPT];
-    auto load_keys = [&]() {
+    auto load_keys = [&](uint4 (&v)[KPT], int split) {
 #pragma unroll
         for (int i = 0; i < KPT; ++i)
-            kv[i] = ldg16u(kc + (size_t)min(j0 + SLOTS * i, n_keys - 1) * row + kh * D + 16 * c);
+            v[i] = ldg16u(kc + (size_t)min(split * kAttnSplit + ks + SLOTS * i, n_keys - 1) * row +
+                          kh * D + 16 * c);
     };
+    __shared__ __attribute__((aligned(16))) uint8_t knew[QKV ? D : 16];    // the new key's codes
     float qv[G][16];
     if constexpr (QKV) {
         // normalized heads: items 0..G-1 the q heads kh*G + g, item G the
@@ -341,9 +361,7 @@ __global__ __launch_bounds__(8 * kAttnSplit / KPT) void attn_scores_kernel(
         // quantized one element per thread.
         constexpr int NI = (G + 1 + NW - 1) / NW;
         __shared__ __attribute__((aligned(16))) uint16_t qs[G][D];
-        __shared__ __attribute__((aligned(16))) uint8_t knew[D];
         const int wave = t >> 6, l = t & 63;
-        const bool last = split == n_splits - 1;
         const int items = last ? G + 1 : G;
         uint32_t rcs = 0;
         if (prep.rope) rcs = reinterpret_cast<const uint32_t*>(prep.rope)[l];
@@ -364,7 +382,7 @@ __global__ __launch_bounds__(8 * kAttnSplit / KPT) void attn_scores_kernel(
                 gb[k] = f32_of_bf16(gm[l + 64]);
             }
         }
-        load_keys();
+        load_keys(kv, split0);
         float cs, sn;
         if (prep.rope) {
             cs = bf16lo(rcs);
@@ -409,14 +427,6 @@ __global__ __launch_bounds__(8 * kAttnSplit / KPT) void attn_scores_kernel(
                 qv[g][2 * e + 1] = bf16hi(d[e]);
             }
         }
-        // the new key (and the clamped indices past it) takes the codes
-        // just computed, not the cache row read before they were written
-        if (last) {
-#pragma unroll
-            for (int i = 0; i < KPT; ++i)
-                if (j0 + SLOTS * i >= n_keys - 1)
-                    kv[i] = *reinterpret_cast<const uint4*>(&knew[16 * c]);
-        }
     } else {
         uint4 qa[G], qb[G];
 #pragma unroll
@@ -425,7 +435,7 @@ __global__ __launch_bounds__(8 * kAttnSplit / KPT) void attn_scores_kernel(
             qa[g] = ldg16u(qp);
             qb[g] = ldg16u(qp + 8);
         }
-        load_keys();
+        load_keys(kv, split0);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const uint4 a = qa[g], b = qb[g];
@@ -437,30 +447,105 @@ __global__ __launch_bounds__(8 * kAttnSplit / KPT) void attn_scores_kernel(
             }
         }
     }
+    // the new key (and the clamped indices past it) takes the codes just
+    // computed, not the cache row read before they were written
+    auto take_new = [&](uint4 (&v)[KPT], int split) {
+#pragma unroll
+        for (int i = 0; i < KPT; ++i)
+            if (split * kAttnSplit + ks + SLOTS * i >= n_keys - 1)
+                v[i] = *reinterpret_cast<const uint4*>(&knew[16 * c]);
+    };
+    if constexpr (QKV && !LOOP)
+        if (last) take_new(kv, split0);
     const float qk_scale = kv_scale[kh] * 0.08838834764831845f;   // sk * f32(1/sqrt(128))
-    float sc[KPT][G];
+    auto score = [&](uint4 (&v)[KPT], int split) {
+        const int j0 = split * kAttnSplit + ks;
+        float sc[KPT][G];
 #pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        float k16[16];
-        decode16(kv[i], k16);
+        for (int i = 0; i < KPT; ++i) {
+            float k16[16];
+            decode16(v[i], k16);
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            float part = 0.0f;
+            for (int g = 0; g < G; ++g) {
+                float part = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) part = __builtin_fmaf(qv[g][e], k16[e], part);
-            part = dpp_add<0xB1>(part);
-            part = dpp_add<0x4E>(part);
-            part = dpp_add<0x141>(part);
-            sc[i][g] = part * qk_scale;
+                for (int e = 0; e < 16; ++e) part = __builtin_fmaf(qv[g][e], k16[e], part);
+                part = dpp_add<0xB1>(part);
+                part = dpp_add<0x4E>(part);
+                part = dpp_add<0x141>(part);
+                sc[i][g] = part * qk_scale;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < KPT; ++i) {
+            const int j = j0 + SLOTS * i;
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                if (c == g && j < n_keys) ws[(size_t)(kh * G + g) * n_keys + j] = sc[i][g];
+        }
+    };
+    if constexpr (!LOOP) {
+        score(kv, split0);
+    } else {
+        uint4 kn[KPT];
+        for (int split = split0; split < n_splits; split += stride) {
+            if (split + stride < n_splits) load_keys(kn, split + stride);
+            if (QKV && split == n_splits - 1) take_new(kv, split);
+            score(kv, split);
+#pragma unroll
+            for (int i = 0; i < KPT; ++i) kv[i] = kn[i];
         }
     }
+}
+
+// Softmax of long contexts: one workgroup per query head turns its scores in
+// the workspace into probabilities p_j = bf16(exp(s_j - m) * (1/sum)) in place,
+// max and sum in attn_values_kernel's orders. Past one pass of keys each of the
+// eight values workgroups of a head would read the scores three times and form
+// every exponential twice; with p at hand they read it once and only multiply
+// (20000 keys: the values kernel 22.5 -> 11.5 us, this one 7.6; the attention
+// 34.2 -> 28.5, 32768 keys 49.9 -> 39.8).
+// The keys sit in registers, RB a thread. Below kSoftmaxMin keys its launch costs
+// more than it saves (8193 keys: 19.4 us without, 21.4 with it), past
+// kSoftmaxMax they no longer fit the registers of 1024 threads and 32
+// workgroups re-reading them are slower (40000 keys: 59 against 64).
+constexpr int kSoftmaxMin = 12 * 1024, kSoftmaxMax = 32 * 1024;
+template <int RB>
+__global__ __launch_bounds__(64 * 16) void attn_softmax_kernel(float* ws, int n_keys)
+{
+    constexpr int NW = 16;
+    float* sh = ws + (size_t)blockIdx.x * n_keys;
+    const int t = threadIdx.x, l = t & 63, wave = t >> 6;
+    __shared__ float red[2][NW];
+    float e[RB];
 #pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        const int j = j0 + SLOTS * i;
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-            if (c == g && j < n_keys) ws[(size_t)(kh * G + g) * n_keys + j] = sc[i][g];
+    for (int k = 0; k < RB; ++k) {
+        const int j = t + 1024 * k;
+        e[k] = j < n_keys ? sh[j] : -3.4e38f;
     }
+    float mx = -3.4e38f;
+#pragma unroll
+    for (int k = 0; k < RB; ++k) mx = fmaxf(mx, e[k]);
+    mx = wave_max64(mx);
+    if (l == 0) red[0][wave] = mx;
+    __syncthreads();
+    float m = red[0][0];
+#pragma unroll
+    for (int v = 1; v < NW; ++v) m = fmaxf(m, red[0][v]);
+    float a = 0.0f;
+#pragma unroll
+    for (int k = 0; k < RB; ++k)
+        if (t + 1024 * k < n_keys) {
+            e[k] = expf(e[k] - m);
+            a += e[k];
+        }
+    a = wave_sum64(a);
+    if (l == 0) red[1][wave] = a;
+    __syncthreads();
+    const float inv = __fdiv_rn(1.0f, sum16_waves(red[1]));
+#pragma unroll
+    for (int k = 0; k < RB; ++k)
+        if (t + 1024 * k < n_keys) sh[t + 1024 * k] = round_bf16(e[k] * inv);
 }
 
 // Values: one workgroup per (query head, 16-dim chunk) over all the keys,
@@ -472,14 +557,18 @@ constexpr int kValWaves = 16;
 constexpr int kValBlocks = 5;
 static_assert(kValWaves == 16, "sum16_waves folds 16 waves");
 
-// ONE: n_keys <= kValWaves * kValBlocks * 64, one pass (its own kernel, so
-// that the register allocation of the common case is its own).
-template <int G, bool ONE>
+// One pass (n_keys <= kValWaves * kValBlocks * 64; its own kernel, so that the
+// register allocation of the common case is its own); several, the scores read
+// again for each phase of the softmax; or several with the probabilities
+// already in ws (attn_softmax_kernel).
+enum ValForm { kValOne, kValMulti, kValProbs };
+template <int G, ValForm FORM>
 __global__ __launch_bounds__(64 * kValWaves) void attn_values_kernel(
     uint16_t* out, const float* ws, const uint8_t* vc, const float* kv_scale, int n_kv,
     int n_keys)
 {
     constexpr int NW = kValWaves, NB = kValBlocks;
+    constexpr bool ONE = FORM == kValOne;
     // kv head kh's workgroups are blockIdx kh + n_kv * i: with 8 kv heads
     // they share one XCD (and its L2) with each other and with the scores
     // kernel's workgroups of kh, which use the same rule
@@ -516,36 +605,39 @@ __global__ __launch_bounds__(64 * kValWaves) void attn_values_kernel(
     // wave (wave_max64 / wave_sum64), then over the 16 waves in LDS (the sum
     // as sum16_waves). With one pass (n_keys <= 16 * 5 * 64) every score is
     // already in registers; longer contexts read the scores again.
-    __shared__ float red[2][NW];
-    float mx = -3.4e38f;
-    if (ONE) {
+    float m = 0.0f, inv = 1.0f;
+    if constexpr (FORM != kValProbs) {
+        __shared__ float red[2][NW];
+        float mx = -3.4e38f;
+        if (ONE) {
 #pragma unroll
-        for (int k = 0; k < NB; ++k)
-            if (kVBlock * (k * NW + wave) + l < n_keys) mx = fmaxf(mx, sa[k]);
-    } else {
-        for (int j = kVBlock * wave + l; j < n_keys; j += kVBlock * NW) mx = fmaxf(mx, sh[j]);
+            for (int k = 0; k < NB; ++k)
+                if (kVBlock * (k * NW + wave) + l < n_keys) mx = fmaxf(mx, sa[k]);
+        } else {
+            for (int j = kVBlock * wave + l; j < n_keys; j += kVBlock * NW) mx = fmaxf(mx, sh[j]);
+        }
+        mx = wave_max64(mx);
+        if (l == 0) red[0][wave] = mx;
+        __syncthreads();
+        m = red[0][0];
+#pragma unroll
+        for (int v = 1; v < NW; ++v) m = fmaxf(m, red[0][v]);
+        float a = 0.0f;
+        if (ONE) {   // sa then holds exp(s_j - m)
+#pragma unroll
+            for (int k = 0; k < NB; ++k)
+                if (kVBlock * (k * NW + wave) + l < n_keys) {
+                    sa[k] = expf(sa[k] - m);
+                    a += sa[k];
+                }
+        } else {
+            for (int j = kVBlock * wave + l; j < n_keys; j += kVBlock * NW) a += expf(sh[j] - m);
+        }
+        a = wave_sum64(a);
+        if (l == 0) red[1][wave] = a;
+        __syncthreads();
+        inv = __fdiv_rn(1.0f, sum16_waves(red[1]));
     }
-    mx = wave_max64(mx);
-    if (l == 0) red[0][wave] = mx;
-    __syncthreads();
-    float m = red[0][0];
-#pragma unroll
-    for (int v = 1; v < NW; ++v) m = fmaxf(m, red[0][v]);
-    float a = 0.0f;
-    if (ONE) {   // sa then holds exp(s_j - m)
-#pragma unroll
-        for (int k = 0; k < NB; ++k)
-            if (kVBlock * (k * NW + wave) + l < n_keys) {
-                sa[k] = expf(sa[k] - m);
-                a += sa[k];
-            }
-    } else {
-        for (int j = kVBlock * wave + l; j < n_keys; j += kVBlock * NW) a += expf(sh[j] - m);
-    }
-    a = wave_sum64(a);
-    if (l == 0) red[1][wave] = a;
-    __syncthreads();
-    const float inv = __fdiv_rn(1.0f, sum16_waves(red[1]));
 
     // p_j = bf16(exp(s_j - m) * inv) (the reference's probability,
     // kernels.mojo:1003-1019); per lane an fma chain over its keys in block
@@ -553,14 +645,15 @@ __global__ __launch_bounds__(64 * kValWaves) void attn_values_kernel(
     float acc[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-    // (have_e: sj holds exp(s_j - m) already)
-    auto consume = [&](int pass, const float (&sj)[NB], const uint4 (&vv)[NB], bool have_e)
+    // (sj holds exp(s_j - m) in the one-pass form, p_j itself in the last)
+    auto consume = [&](int pass, const float (&sj)[NB], const uint4 (&vv)[NB])
         __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
             const int j = kVBlock * ((pass * NB + k) * NW + wave) + l;
             if (j < n_keys) {
-                const float pj = round_bf16((have_e ? sj[k] : expf(sj[k] - m)) * inv);
+                const float pj = FORM == kValProbs ? sj[k]
+                                 : round_bf16((ONE ? sj[k] : expf(sj[k] - m)) * inv);
                 float v16[16];
                 decode16(vv[k], v16);
 #pragma unroll
@@ -569,15 +662,15 @@ __global__ __launch_bounds__(64 * kValWaves) void attn_values_kernel(
         }
     };
     if (ONE) {
-        consume(0, sa, va, true);
+        consume(0, sa, va);
     } else {
         issue(0, sa, va);
         for (int p = 0; p < n_pass; p += 2) {
             if (p + 1 < n_pass) issue(p + 1, sb, vb);
-            consume(p, sa, va, false);
+            consume(p, sa, va);
             if (p + 1 >= n_pass) break;
             if (p + 2 < n_pass) issue(p + 2, sa, va);
-            consume(p + 1, sb, vb, false);
+            consume(p + 1, sb, vb);
         }
     }
 
@@ -711,20 +804,31 @@ hipError_t launch_attention(uint16_t* out, const uint16_t* q, const uint8_t* kc,
                             const QkvPrep& prep = QkvPrep{})
 {
     const int splits = (n_keys + kAttnSplit - 1) / kAttnSplit;
-    const int blocks = n_kv * splits;
-    constexpr int NT = 8 * kAttnSplit / kAttnKPT;
-    if (prep.qkv)
-        attn_scores_kernel<G, true, kAttnKPT><<<blocks, NT, 0, s>>>(ws, q, kc, kv_scale, n_kv,
-                                                                   n_keys, splits, prep);
-    else
-        attn_scores_kernel<G, false, kAttnKPT><<<blocks, NT, 0, s>>>(ws, q, kc, kv_scale, n_kv,
-                                                                    n_keys, splits, prep);
-    if (n_keys <= kValWaves * kValBlocks * kVBlock)
-        attn_values_kernel<G, true><<<n_kv * G * 8, 64 * kValWaves, 0, s>>>(out, ws, vc, kv_scale,
-                                                                            n_kv, n_keys);
-    else
-        attn_values_kernel<G, false><<<n_kv * G * 8, 64 * kValWaves, 0, s>>>(out, ws, vc, kv_scale,
-                                                                             n_kv, n_keys);
+    const int per_kv = std::max(1, kAttnSlots<G> / n_kv);    // workgroups that fit at once
+    constexpr int NT = 8 * kAttnSplit / kAttnKPT<G>;
+    const int stride = std::min(splits, per_kv), blocks = n_kv * stride;
+    auto scores = [&](auto qkv, auto loop) {
+        attn_scores_kernel<G, decltype(qkv)::value, kAttnKPT<G>, decltype(loop)::value>
+            <<<blocks, NT, 0, s>>>(ws, q, kc, kv_scale, n_kv, n_keys, splits, stride, prep);
+    };
+    if (prep.qkv) {
+        if (splits > per_kv) scores(std::true_type{}, std::true_type{});
+        else scores(std::true_type{}, std::false_type{});
+    } else {
+        if (splits > per_kv) scores(std::false_type{}, std::true_type{});
+        else scores(std::false_type{}, std::false_type{});
+    }
+    const dim3 vgrid(n_kv * G * 8);
+    constexpr int VT = 64 * kValWaves;
+    if (n_keys <= kValWaves * kValBlocks * kVBlock) {
+        attn_values_kernel<G, kValOne><<<vgrid, VT, 0, s>>>(out, ws, vc, kv_scale, n_kv, n_keys);
+    } else if (n_keys > kSoftmaxMin && n_keys <= kSoftmaxMax) {
+        if (n_keys <= 20 * 1024) attn_softmax_kernel<20><<<n_kv * G, 1024, 0, s>>>(ws, n_keys);
+        else attn_softmax_kernel<32><<<n_kv * G, 1024, 0, s>>>(ws, n_keys);
+        attn_values_kernel<G, kValProbs><<<vgrid, VT, 0, s>>>(out, ws, vc, kv_scale, n_kv, n_keys);
+    } else {
+        attn_values_kernel<G, kValMulti><<<vgrid, VT, 0, s>>>(out, ws, vc, kv_scale, n_kv, n_keys);
+    }
     return hipGetLastError();
 }
 

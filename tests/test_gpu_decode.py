@@ -235,6 +235,23 @@ def test_attention_max_context_exact():
     assert np.all(got == 1.25), np.unique(got)[:8]
 
 
+@pytest.mark.parametrize("n", [8192, 8193, 12288, 12289, 20480, 20481, 32768, 32769])
+def test_attention_long_forms_vs_oracle(n):
+    # Where the long-context forms change hands: one split per scores workgroup
+    # up to 8192 keys with 8 kv heads, more past it; the softmax kernel and the
+    # values from its probabilities from 12289 to 32768 keys (20 keys a thread
+    # up to 20480, else 32), the multi-pass values kernel on either side.
+    test_attention_vs_oracle(n)
+
+
+@pytest.mark.parametrize("nh,nkv,pos", [(32, 8, 8191), (32, 8, 8192), (32, 8, 20001), (8, 8, 16384),
+                                        (8, 4, 16400), (16, 2, 5000), (32, 4, 33000)])
+def test_attention_qkv_long_matches_separate_ops(nh, nkv, pos):
+    # The fused form with several splits per scores workgroup: the newest key in
+    # a workgroup's first, middle or last split, 1, 2, 4 and 8 query heads.
+    test_attention_qkv_matches_separate_ops(pos, nh, nkv)
+
+
 def test_attention_rejects_long_context_and_small_workspace():
     z = torch.zeros(16, dtype=torch.uint8, device="cuda")
     with pytest.raises(HephError):
