@@ -104,31 +104,6 @@ __device__ __forceinline__ void store_codes(uint8_t* p, const uint32_t* cd)
     }
 }
 
-// Max over each aligned run of LPR lanes, unsigned integers, left in every
-// lane of the run: DPP within each 16-lane row, then gfx950's lane swaps
-// (v_permlane16_swap pairs rows 0-1 and 2-3, v_permlane32_swap the two
-// halves), which stay in the VALU instead of going through LDS.
-template <int LPR>
-__device__ __forceinline__ uint32_t lanes_max_u(uint32_t m)
-{
-    auto dpp = [](uint32_t x, auto ctrl) {
-        return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, decltype(ctrl)::value, 0xf, 0xf, false);
-    };
-    m = max(m, dpp(m, std::integral_constant<int, 0xB1>{}));
-    m = max(m, dpp(m, std::integral_constant<int, 0x4E>{}));
-    if constexpr (LPR >= 8) m = max(m, dpp(m, std::integral_constant<int, 0x141>{}));
-    if constexpr (LPR >= 16) m = max(m, dpp(m, std::integral_constant<int, 0x140>{}));
-    if constexpr (LPR >= 32) {
-        const auto r = __builtin_amdgcn_permlane16_swap(m, m, false, false);
-        m = max((uint32_t)r[0], (uint32_t)r[1]);
-    }
-    if constexpr (LPR == 64) {
-        const auto r = __builtin_amdgcn_permlane32_swap(m, m, false, false);
-        m = max((uint32_t)r[0], (uint32_t)r[1]);
-    }
-    return m;
-}
-
 // Four floats -> four E4M3FN codes (byte i = code of value i), RNE. The
 // first conversion writes the low half of a register whose other half the
 // second one overwrites, so its previous contents do not matter.

@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "group_scale.h"
 
 namespace heph {
@@ -139,6 +141,31 @@ __device__ __forceinline__ float bf16_bits_f32(uint32_t b) { return __uint_as_fl
 __device__ __forceinline__ uint32_t shfl_xor_u(uint32_t v, int o)
 {
     return (uint32_t)__shfl_xor((int)v, o);
+}
+
+// Max over each aligned run of LPR lanes, unsigned integers, left in every
+// lane of the run: DPP within each 16-lane row, then gfx950's lane swaps
+// (v_permlane16_swap pairs rows 0-1 and 2-3, v_permlane32_swap the two
+// halves), which stay in the VALU instead of going through LDS.
+template <int LPR>
+__device__ __forceinline__ uint32_t lanes_max_u(uint32_t m)
+{
+    auto dpp = [](uint32_t x, auto ctrl) {
+        return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, decltype(ctrl)::value, 0xf, 0xf, false);
+    };
+    m = max(m, dpp(m, std::integral_constant<int, 0xB1>{}));
+    m = max(m, dpp(m, std::integral_constant<int, 0x4E>{}));
+    if constexpr (LPR >= 8) m = max(m, dpp(m, std::integral_constant<int, 0x141>{}));
+    if constexpr (LPR >= 16) m = max(m, dpp(m, std::integral_constant<int, 0x140>{}));
+    if constexpr (LPR >= 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+        m = max((uint32_t)r[0], (uint32_t)r[1]);
+    }
+    if constexpr (LPR == 64) {
+        const auto r = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+        m = max((uint32_t)r[0], (uint32_t)r[1]);
+    }
+    return m;
 }
 
 // Eight bf16 times inv -> eight codes in two dwords.

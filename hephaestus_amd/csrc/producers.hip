@@ -13,6 +13,8 @@
 // HEPH_FLAG_SKIP_QUANT: one launch and one read of the bf16 activations
 // fewer per linear, and the normalized (activated) bf16 row is never
 // written.
+#include <algorithm>
+
 #include "../../include/hephdecode.h"
 #include "heph_kernels.h"
 
@@ -72,51 +74,117 @@ __device__ __forceinline__ void quant_row_from_lds(const uint16_t* yrow, int col
         *reinterpret_cast<uint2*>(q + k) = quant8(*reinterpret_cast<const uint4*>(yrow + k), inv);
 }
 
-// One 256-thread workgroup per row. The norm is heph_rmsnorm's: thread t
-// owns elements t, t + 256, ... and sums their squares in that order (fma),
-// the 256 sums fold as fold256_wave0 does, and y = bf16(gamma * bf16(x * r)).
-// y goes to LDS instead of global memory (dynamic, 2 * cols bytes, so that
-// short rows leave room for more workgroups per CU); then the row is
-// quantized.
-template <int PER>
-__global__ __launch_bounds__(256) void rmsnorm_quant_kernel(uint8_t* q, float* scales,
-                                                            const uint16_t* in,
-                                                            const uint16_t* gamma, int cols,
-                                                            float eps, int group_k)
+// One workgroup per row. The norm is heph_rmsnorm's: thread t < 256 sums the
+// squares of elements t, t + 256, ... in that order (fma), the 256 sums fold as
+// fold256_wave0 does, and y = bf16(gamma * bf16(x * r)). A row of a prefill
+// batch is a few KB, so the kernel is a chain of latencies; it is kept to one
+// round of 16-byte loads (PPT pieces of 8 elements a thread, the row's and
+// gamma's in flight together), one staging of the row in LDS for the sums in
+// their order, and two barriers: a thread then normalizes the pieces it still
+// holds, and sixteen neighbouring lanes hold a whole 1x128 group, quantized
+// where it is. MI355X, graph-replayed, against 2-byte
+// loads of elements t, t + 256, .. and a second staging of y for the groups:
+// 512 rows of 2560 6.4 -> 4.3 us, 64 of 4096 7.5 -> 3.7, 4096 of 2560 19.7 ->
+// 14.5.
+template <int PPT>
+__global__ __launch_bounds__(1024) void rmsnorm_quant_kernel(uint8_t* q, float* scales,
+                                                             const uint16_t* in,
+                                                             const uint16_t* gamma, int cols,
+                                                             float eps, int group_k)
+{
+    __shared__ float red[256];
+    __shared__ uint32_t redm[16];
+    extern __shared__ __attribute__((aligned(16))) uint16_t xrow[];
+    const int t = threadIdx.x, nt = blockDim.x, np = cols / 8;
+    const uint16_t* x = in + (size_t)blockIdx.x * cols;
+    uint4 xv[PPT], gv[PPT];
+#pragma unroll
+    for (int k = 0; k < PPT; ++k) {
+        const int p = t + k * nt;
+        xv[k] = gv[k] = make_uint4(0, 0, 0, 0);
+        if (p < np) {
+            xv[k] = ldg16u(x + 8 * p);
+            gv[k] = ldg16u(gamma + 8 * p);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < PPT; ++k)
+        if (t + k * nt < np) *reinterpret_cast<uint4*>(xrow + 8 * (t + k * nt)) = xv[k];
+    __syncthreads();
+    float ss = 0.0f;
+    if (t < 256) {
+#pragma unroll 8
+        for (int i = t; i < cols; i += 256) {
+            const float v = f32b(xrow[i]);
+            ss = __builtin_fmaf(v, v, ss);
+        }
+    }
+    const float r = rms_inv(fold256_every_wave(ss, red), cols, eps);
+    uint4 y[PPT];
+#pragma unroll
+    for (int k = 0; k < PPT; ++k) {
+        const uint32_t xd[4] = {xv[k].x, xv[k].y, xv[k].z, xv[k].w};
+        const uint32_t gd[4] = {gv[k].x, gv[k].y, gv[k].z, gv[k].w};
+        uint32_t yd[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+            yd[d] = (uint32_t)f32_to_bf16(bf16lo(gd[d]) * rbf16(bf16lo(xd[d]) * r)) |
+                    ((uint32_t)f32_to_bf16(bf16hi(gd[d]) * rbf16(bf16hi(xd[d]) * r)) << 16);
+        y[k] = make_uint4(yd[0], yd[1], yd[2], yd[3]);
+    }
+    uint8_t* qr = q + (size_t)blockIdx.x * cols;
+    if (group_k == kChunk) {
+        // (cols % 128 == 0: a team of 16 lanes is whole or has no piece)
+        float* sr = scales + (size_t)blockIdx.x * (cols / kChunk);
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) {
+            const int p = t + k * nt;
+            uint32_t mb = absmax_bits8(y[k]);
+            if (mb > 0x7F80u) mb = absmax_bits8_skip_nan(y[k]);    // this lane holds a NaN
+            mb = lanes_max_u<16>(mb);
+            float sc, inv;
+            group_scale(bf16_bits_f32(mb), sc, inv);
+            if (p < np) {
+                *reinterpret_cast<uint2*>(qr + 8 * p) = quant8(y[k], inv);
+                if ((p & 15) == 0) sr[p >> 4] = sc;
+            }
+        }
+        return;
+    }
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < PPT; ++k) m = absmax_bits8_skip_nan(y[k], m);
+    m = lanes_max_u<64>(m);
+    if ((t & 63) == 0) redm[t >> 6] = m;
+    __syncthreads();
+    for (int w = 0; w < nt / 64; ++w) m = max(m, redm[w]);
+    float sc, inv;
+    group_scale(bf16_bits_f32(m), sc, inv);
+    if (t == 0) scales[blockIdx.x] = sc;
+#pragma unroll
+    for (int k = 0; k < PPT; ++k)
+        if (t + k * nt < np) *reinterpret_cast<uint2*>(qr + 8 * (t + k * nt)) = quant8(y[k], inv);
+}
+
+// The same for a row or gamma that is not 16-byte aligned: element loads, y
+// staged in LDS and quantized from there.
+__global__ __launch_bounds__(256) void rmsnorm_quant_unaligned_kernel(
+    uint8_t* q, float* scales, const uint16_t* in, const uint16_t* gamma, int cols, float eps,
+    int group_k)
 {
     __shared__ float red[256];
     __shared__ float res;
     extern __shared__ __attribute__((aligned(16))) uint16_t yrow[];
     const uint16_t* x = in + (size_t)blockIdx.x * cols;
     const int t = threadIdx.x;
-    if constexpr (PER > 0) {
-        float v[PER], g[PER];
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-            const int i = t + e * 256;
-            v[e] = i < cols ? f32b(x[i]) : 0.0f;
-            g[e] = i < cols ? f32b(gamma[i]) : 0.0f;
-        }
-        float ss = 0.0f;
-#pragma unroll
-        for (int e = 0; e < PER; ++e)
-            if (t + e * 256 < cols) ss = __builtin_fmaf(v[e], v[e], ss);
-        const float r = rms_inv(fold256_wave0(ss, red, &res), cols, eps);
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-            const int i = t + e * 256;
-            if (i < cols) yrow[i] = f32_to_bf16(g[e] * rbf16(v[e] * r));
-        }
-    } else {
-        float ss = 0.0f;
-        for (int i = t; i < cols; i += 256) {
-            const float v = f32b(x[i]);
-            ss = __builtin_fmaf(v, v, ss);
-        }
-        const float r = rms_inv(fold256_wave0(ss, red, &res), cols, eps);
-        for (int i = t; i < cols; i += 256)
-            yrow[i] = f32_to_bf16(f32b(gamma[i]) * rbf16(f32b(x[i]) * r));
+    float ss = 0.0f;
+    for (int i = t; i < cols; i += 256) {
+        const float v = f32b(x[i]);
+        ss = __builtin_fmaf(v, v, ss);
     }
+    const float r = rms_inv(fold256_wave0(ss, red, &res), cols, eps);
+    for (int i = t; i < cols; i += 256)
+        yrow[i] = f32_to_bf16(f32b(gamma[i]) * rbf16(f32b(x[i]) * r));
     __syncthreads();
     quant_row_from_lds(yrow, cols, group_k, q + (size_t)blockIdx.x * cols,
                        scales + (size_t)blockIdx.x * (cols / group_k));
@@ -201,20 +269,18 @@ int heph_rmsnorm_quant_fp8(uint8_t* q, float* scales, const uint16_t* x_bf16,
     if (!a16(q)) return HEPH_ERR_ALIGN;
     if (int st = check_device()) return st;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int per = (cols + 255) / 256;
     const size_t lds = (size_t)cols * 2;
-    if (per <= 10)
-        rmsnorm_quant_kernel<10><<<rows, 256, lds, s>>>(q, scales, x_bf16, gamma_bf16, cols, eps,
-                                                      group_k);
-    else if (per <= 16)
-        rmsnorm_quant_kernel<16><<<rows, 256, lds, s>>>(q, scales, x_bf16, gamma_bf16, cols, eps,
-                                                      group_k);
-    else if (per <= 40)
-        rmsnorm_quant_kernel<40><<<rows, 256, lds, s>>>(q, scales, x_bf16, gamma_bf16, cols, eps,
+    const int np = cols / 8;      // 16-byte pieces; 16384 / 8 = two per thread
+    const int nt = std::min(1024, std::max(256, (np + 63) / 64 * 64));
+    if (!a16(x_bf16) || !a16(gamma_bf16))
+        rmsnorm_quant_unaligned_kernel<<<rows, 256, lds, s>>>(q, scales, x_bf16, gamma_bf16, cols,
+                                                              eps, group_k);
+    else if (np <= nt)
+        rmsnorm_quant_kernel<1><<<rows, nt, lds, s>>>(q, scales, x_bf16, gamma_bf16, cols, eps,
                                                       group_k);
     else
-        rmsnorm_quant_kernel<0><<<rows, 256, lds, s>>>(q, scales, x_bf16, gamma_bf16, cols, eps,
-                                                     group_k);
+        rmsnorm_quant_kernel<2><<<rows, nt, lds, s>>>(q, scales, x_bf16, gamma_bf16, cols, eps,
+                                                      group_k);
     return hipGetLastError() == hipSuccess ? HEPH_OK : HEPH_ERR_LAUNCH;
 }
 

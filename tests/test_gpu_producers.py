@@ -46,6 +46,30 @@ def test_rmsnorm_quant_bit_exact(rows, cols, scale, group):
     assert np.array_equal(s1.cpu().numpy().reshape(so.shape), so)
 
 
+@pytest.mark.parametrize("cols", [128, 2048, 2176, 8192, 8320, 16384])
+@pytest.mark.parametrize("group", ["g128", "token"])
+@pytest.mark.parametrize("off", [0, 1])
+def test_rmsnorm_quant_piece_edges_and_alignment(cols, group, off):
+    # One and two 16-byte pieces a thread (256 threads up to 2048 columns, 1024
+    # from 8192 on), and a row and gamma that start off 16-byte alignment: the
+    # norm and the quantizer on their own give the same bytes.
+    g, rows = (128 if group == "g128" else cols), 3
+    x = torch.randn(rows * cols + off, device="cuda").to(torch.bfloat16)[off:]
+    x[5], x[cols + 7] = float("nan"), 300.0
+    gam = torch.randn(cols + off, device="cuda").to(torch.bfloat16)[off:]
+    q1 = torch.zeros(rows * cols, dtype=torch.uint8, device="cuda")
+    s1 = torch.zeros(rows * (cols // g), dtype=torch.float32, device="cuda")
+    HK.rmsnorm_quant_fp8(q1, s1, x, gam, rows, cols, 1e-6, group_k=g)
+    y = torch.empty(rows, cols, dtype=torch.bfloat16, device="cuda")
+    DEC.rmsnorm(y, x.view(rows, cols), gam)
+    q2, s2 = torch.zeros_like(q1), torch.zeros_like(s1)
+    HK.quantize_act_rows_fp8(q2, s2, y, rows, cols, group_k=g)
+    torch.cuda.synchronize()
+    assert torch.equal(q1[cols:], q2[cols:]) and torch.equal(s1, s2)
+    # row 0 is all NaN (its factor is): codes up to the sign of NaN
+    assert torch.equal(q1[:cols] & 0x7F, q2[:cols] & 0x7F)
+
+
 def test_rmsnorm_quant_config3_m4096_codes_vs_oracle():
     rows, cols = 4096, 2560
     x = rows_bf16(33, rows, cols, outliers=1e-3)
