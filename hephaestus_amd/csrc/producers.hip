@@ -203,7 +203,9 @@ __device__ __forceinline__ uint4 swiglu8(const uint4& g, const uint4& u)
 
 // 1x128 groups: one 16-lane team per group of one row, 8 elements a lane,
 // the SwiGLU values computed in registers and quantized as
-// quant_g128_kernel does.
+// quant_g128_kernel does. 6 bytes of traffic an element against ~25
+// instructions (silu_bf16; ~60 with expf and an IEEE division, which bound the
+// kernel): 512 rows of 9728 10.2 -> 7.6 us, 4096 rows 57.3 -> 39.9 (6.0 TB/s).
 __global__ __launch_bounds__(256) void silu_mul_quant_g128_kernel(
     uint8_t* __restrict__ q, float* __restrict__ scales, const uint16_t* __restrict__ gate,
     const uint16_t* __restrict__ up, int n, long ld, long n_groups)

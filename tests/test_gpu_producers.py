@@ -108,6 +108,30 @@ def test_silu_mul_quant_bit_exact(rows, n, ld, group):
     assert torch.equal(q1, q2)
 
 
+def test_silu_mul_every_bf16_gate():
+    # All 65536 gate values, bit for bit bf16(g / (1 + exp(-g))) by torch's f32
+    # exp and division (NaN as NaN), through silu_mul and, for one up value,
+    # the bf16 product; the quantizing form gives the codes of those values.
+    g = torch.arange(65536, dtype=torch.int32, device="cuda").to(torch.int16).view(torch.bfloat16)
+    gf = g.float()
+    s = (gf / (1.0 + torch.exp(-gf))).to(torch.bfloat16)
+    for u in (1.0, -0.7109375):
+        up = torch.full_like(g, u)
+        out = torch.empty_like(g)
+        DEC.silu_mul(out, g, up, 65536)
+        want = (s.float() * up.float()).to(torch.bfloat16)
+        torch.cuda.synchronize()
+        ok = (out.view(torch.int16) == want.view(torch.int16)) | (out.isnan() & want.isnan())
+        bad = torch.nonzero(~ok).flatten()
+        assert bad.numel() == 0, (u, gf[bad[:8]].tolist(), out[bad[:8]].tolist())
+        q1, s1 = HK.workspace(512, 128)
+        HK.silu_mul_quant_fp8(q1, s1, g, up, 512, 128)
+        q2, s2 = HK.workspace(512, 128)
+        HK.quantize_act_rows_fp8(q2, s2, out, 512, 128)
+        torch.cuda.synchronize()
+        assert torch.equal(q1, q2) and torch.equal(s1, s2)
+
+
 def test_prefill_path_with_producers_equals_unfused():
     # RMSNorm -> qkv and SwiGLU -> down at M = 512: the producer's codes fed
     # to the linear with SKIP_QUANT give the unfused path's bits.
