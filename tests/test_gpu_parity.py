@@ -832,6 +832,29 @@ def test_weight_quant_vs_oracle(N, K):
     assert codes_match(q.cpu().numpy(), qo)
 
 
+@pytest.mark.parametrize("exp", [-32, -30, 0, 120])
+def test_weight_quant_quotients_are_the_ieee_ones(exp):
+    # One block per amax mantissa (128 of them, x 2^exp), holding every bf16
+    # mantissa at the 16 exponents down from the amax's, both signs, and both
+    # zeros: the codes are those of the division. At 2^-32 some blocks' scale
+    # is below the 1e-12 floor, at 2^-30 it is just above.
+    from hephaestus_amd.weights import quantize_weight_fp8
+    mant = np.arange(128, dtype=np.int32)
+    blocks = np.zeros((128, 128, 128), np.uint16)
+    for b in range(128):
+        bits = ((127 + exp - np.arange(32)[:, None] // 2) << 7) | mant[None, :]
+        bits = np.minimum(bits, ((127 + exp) << 7) | b).astype(np.uint16)
+        bits[1::2] |= 0x8000
+        blocks[b, :32] = bits
+        blocks[b, 33] = 0x8000                                   # -0
+    w = blocks.transpose(1, 0, 2).reshape(128, 128 * 128).copy()
+    q, s = quantize_weight_fp8(dev(w))
+    torch.cuda.synchronize()
+    qo, so = O.quant_weight(f32_of_bf16(w), 128, 128)
+    assert np.array_equal(s.cpu().numpy(), so)
+    assert np.array_equal(q.cpu().numpy(), qo)
+
+
 def test_graph_capture_replays_match_eager():
     # The linear launches are capturable (no memsets, no host sync); every
     # replay, with eager work and syncs between, equals the eager result.
