@@ -358,8 +358,10 @@ static double ring_estimate(int M, int N, int K, const RingCost& rc, int s)
 }
 
 // Tile and K splits of the large-M GEMM: the pair with the least estimated
-// time, splitting only when allowed, into at most 8 splits of at least 4
-// chunks; ties go to the earlier tile of kTileCost, then to fewer splits.
+// time, splitting into at most 8 splits of at least 4 chunks, and only where
+// `scratch` bytes hold the fp32 partials (a ring tile then takes fewer splits,
+// a large tile none: a buffer sized for other rows may be any size); ties go
+// to the earlier tile of kTileCost, then to fewer splits.
 // A forced tile height (gemm_bm) or width (gemm_bn) keeps only the tiles
 // that have it. per_token (nothing varies along K): the large tiles do not
 // split.
@@ -368,59 +370,68 @@ static double ring_estimate(int M, int N, int K, const RingCost& rc, int s)
 // that: over the 47 shapes of its fit the choice then ran at 0.80 (block
 // scales) and 0.69 (per-token) of the large tiles' time, 1.02 at worst (0.8 to
 // 1.0: up to 1.19; from M = 470 on the two run alike). Past K = 4096 the ring
-// always splits where it may: one workgroup's chain of chunks is then longer
-// than a reduction.
-GemmPlan gemm_plan(int M, int N, int K, bool can_split, int forced_bm, int forced_bn,
+// splits first: one workgroup's chain of chunks is then longer than a
+// reduction.
+GemmPlan gemm_plan(int M, int N, int K, size_t scratch, int forced_bm, int forced_bn,
                    bool per_token)
 {
+    const auto fits = [&](int s) { return s == 1 || (size_t)s * M * N * 4 <= scratch; };
     // MI355X's 256 CUs, not the visible count: the plan (and the K-split
     // summation order with it) does not change under a CU mask or partition
     const long cus = kPlanCUs;
     const int KC = K / kChunk;
     GemmPlan best{0, 0, 1, false};
     double best_t = -1.0;
-    for (const auto& tc : kTileCost) {
-        // 64 x 192 only where its fit holds (M >= 256): below, the K-split
-        // plans of the small-M routes stay with the tiles they were measured on
-        if (tc.bm == 64 && tc.bn == 192 && M < 256 && forced_bn != 192) continue;
-        if (forced_bm >= 64 && tc.bm != forced_bm) continue;
-        if (forced_bn && tc.bn != forced_bn) continue;
-        for (int s = 1; s <= (can_split && !per_token ? 8 : 1); ++s) {
-            if (s > 1 && KC / s < 4) break;
-            const double t = gemm_estimate(M, N, K, tc, s, cus);
-            if (best_t < 0.0 || t < best_t) {
-                best_t = t;
-                best = GemmPlan{tc.bm, tc.bn, s, false};
+    const auto large = [&](int max_splits) {
+        best = GemmPlan{0, 0, 1, false};
+        best_t = -1.0;
+        for (const auto& tc : kTileCost) {
+            // 64 x 192 only where its fit holds (M >= 256): below, the K-split
+            // plans of the small-M routes stay with the tiles they were measured on
+            if (tc.bm == 64 && tc.bn == 192 && M < 256 && forced_bn != 192) continue;
+            if (forced_bm >= 64 && tc.bm != forced_bm) continue;
+            if (forced_bn && tc.bn != forced_bn) continue;
+            for (int s = 1; s <= max_splits; ++s) {
+                if (s > 1 && KC / s < 4) break;
+                const double t = gemm_estimate(M, N, K, tc, s, cus);
+                if (best_t < 0.0 || t < best_t) {
+                    best_t = t;
+                    best = GemmPlan{tc.bm, tc.bn, s, false};
+                }
             }
         }
-    }
+    };
+    large(per_token ? 1 : 8);
+    if (!fits(best.splits)) large(1);
     if (best.bm == 0) best = GemmPlan{forced_bm >= 64 ? forced_bm : 256, 256, 1, false};
     if (M <= 32 || M >= (per_token ? 1024 : 512) || forced_bm || forced_bn) return best;
     best_t *= 0.8;
-    for (const auto& rc : kRingCost) {
-        for (int s = can_split && K > 4096 ? 2 : 1; s <= (can_split ? 8 : 1); ++s) {
-            if (s > 1 && KC / s < 4) break;
-            const double t = ring_estimate(M, N, K, rc, s);
-            if (t < best_t) {
-                best_t = t;
-                best = GemmPlan{rc.bm, rc.bn, s, true};
+    const auto ring = [&](int s0, int s1) {
+        for (const auto& rc : kRingCost) {
+            for (int s = s0; s <= s1 && fits(s); ++s) {
+                if (s > 1 && KC / s < 4) break;
+                const double t = ring_estimate(M, N, K, rc, s);
+                if (t < best_t) {
+                    best_t = t;
+                    best = GemmPlan{rc.bm, rc.bn, s, true};
+                }
             }
         }
-    }
+    };
+    ring(K > 4096 ? 2 : 1, 8);
+    if (!best.ring && best.splits == 1) ring(1, 1);
     return best;
 }
 
 bool gemm_splits_ready(const Fp8Operands& op)
 {
-    if (!op.part) return false;
-    const int s = gemm_plan(op.M, op.N, op.K, true, op.tune.gemm_bm, op.tune.gemm_bn,
-                            op.s_step == 0).splits;
-    return s > 1 && op.part_bytes >= (size_t)s * op.M * op.N * 4;
+    return gemm_plan(op.M, op.N, op.K, op.part ? op.part_bytes : 0, op.tune.gemm_bm,
+                     op.tune.gemm_bn, op.s_step == 0).splits > 1;
 }
 
 size_t gemm_split_bytes(int M, int N, int K)
 {
-    const int s = gemm_plan(M, N, K, true).splits;
+    const int s = gemm_plan(M, N, K, SIZE_MAX).splits;
     return s > 1 ? (size_t)s * M * N * 4 : 0;
 }
 
@@ -435,9 +446,8 @@ hipError_t launch_fp8_gemm(const Fp8Operands& op, hipStream_t stream,
     const bool small_offsets = (long)op.M * op.K < (1L << 31) && (long)op.N * op.K < (1L << 31);
     const bool force_128 = op.tune.gemm_bm == 1;
     if (small_offsets && !force_128) {
-        // K splits when the caller's scratch holds their partials.
         Fp8Operands o = op;
-        const GemmPlan plan = gemm_plan(o.M, o.N, o.K, gemm_splits_ready(o), o.tune.gemm_bm,
+        const GemmPlan plan = gemm_plan(o.M, o.N, o.K, o.part ? o.part_bytes : 0, o.tune.gemm_bm,
                                         o.tune.gemm_bn, o.s_step == 0);
         o.splits = plan.splits;
         const bool sk = o.splits > 1;

@@ -128,14 +128,14 @@ hipError_t launch_fp8_gemm(const Fp8Operands& op, hipStream_t stream,
                            const LaunchTiming& t, const char** name);
 
 // Tile (bm x bn; ring: a tile of gemm_ring.h, else of gemm_big.h) and K
-// splits (1 = none) of the GEMM for M x N x K, splits only if can_split;
-// forced_bm / forced_bn keep only the large tiles of that height / width (0 =
+// splits (1 = none) of the GEMM for M x N x K, splits only where `scratch`
+// bytes hold their partials; forced_bm / forced_bn keep only the large tiles of that height / width (0 =
 // automatic); per_token: per-token and per-channel scales.
 struct GemmPlan {
     int bm, bn, splits;
     bool ring;
 };
-GemmPlan gemm_plan(int M, int N, int K, bool can_split, int forced_bm = 0, int forced_bn = 0,
+GemmPlan gemm_plan(int M, int N, int K, size_t scratch, int forced_bm = 0, int forced_bn = 0,
                    bool per_token = false);
 // Scratch bytes for the partials of the split plan (0 when it does not
 // split), and whether op's scratch (part) holds them for a plan of more

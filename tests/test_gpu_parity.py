@@ -1426,6 +1426,28 @@ def test_ring_tiles_vs_oracle(tile, M, N, K, mode, out, resid):
     assert np.array_equal(q_ws[: M * K].cpu().numpy().reshape(M, K), qo)
 
 
+@pytest.mark.parametrize("M,cap", [(73, 128), (96, 128)])
+def test_ring_splits_fit_a_buffer_of_other_rows(M, cap):
+    # A workspace sized for 128 rows of down_proj holds fewer partials than the
+    # plan of 73 .. 96 rows would take: K splits into as many as fit, nothing
+    # past the buffer's end is written.
+    N, K = 2560, 9728
+    ia, qa = lattice(M, K, 8100 + M)
+    iw, qw = lattice(N, K, 8101)
+    ref = (ia.astype(np.float64) @ iw.astype(np.float64).T) * 0.0625 * 2.0 ** -5
+    need = L.lib().heph_fp8_linear_ws_bytes(cap, N, K)
+    assert L.lib().heph_fp8_linear_ws_bytes(M, N, K) > need
+    buf = torch.full((need + 4096,), 0xA5, dtype=torch.uint8, device="cuda")
+    q_ws = buf[:need]
+    s_ws = torch.full((cap * (K // 128),), 2.0 ** -3, dtype=torch.float32, device="cuda")
+    q_ws[: M * K].copy_(dev(qa.reshape(-1)))
+    c, _, _ = run_linear(qw, np.full((-(-N // 128), K // 128), 2.0 ** -2, np.float32), None, M=M,
+                         N=N, K=K, group_k=128, skip_quant=True, q_ws=q_ws, s_ws=s_ws)
+    assert HK.last_kernel().endswith("_splitk"), HK.last_kernel()
+    assert np.array_equal(host_bf16(c), bf16_of(ref.astype(np.float32)))
+    assert bool((buf[need:] == 0xA5).all())
+
+
 @pytest.mark.parametrize("tile,M,N,K", RING_CASES)
 def test_ring_tiles_exact_integer(tile, M, N, K):
     # Every partial sum is an integer below 2^24 times a power of two: bit for
