@@ -132,7 +132,7 @@ def attention_qkv_fp8kv(out, qkv, q_gamma, k_gamma, k_cache, v_cache, kv_scale, 
                         eps: float = 1e-6, ws: torch.Tensor | None = None,
                         rope: torch.Tensor | None = None) -> None:
     """qk_norm_rope_kv into cache key pos, then attention_fp8kv over pos + 1
-    keys, in the attention's two launches (the same out and cache bytes;
+    keys, in the attention's own launches (the same out and cache bytes;
     q in qkv is not rotated in place). rope: a rope_table of more than pos
     rows for this theta, or None to compute pos's cos/sin in the call."""
     if ws is None:

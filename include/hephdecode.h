@@ -68,10 +68,11 @@ int heph_qk_norm_rope_kv(void* qkv_bf16, const void* q_gamma, const void* k_gamm
 /*
  * One query token over n_keys cached keys: out[h] = sum_j p_j * v_j with
  * p = bf16(softmax(q.k_j * sk / sqrt(128))), K and V E4M3 codes in the
- * layouts above scaled by kv_scale (K entries, then V), in two launches.
+ * layouts above scaled by kv_scale (K entries, then V), in two launches (a
+ * softmax between them from 12289 to 32768 keys).
  * n_heads / n_kv_heads (query heads per kv head) must be 1, 2, 4 or 8.
  * ws: device scratch of heph_attention_ws_bytes(n_heads, n_keys) bytes
- * (the fp32 scores), 16-byte aligned.
+ * (the fp32 scores, which the call may overwrite), 16-byte aligned.
  * Replaces attention (src/hephaestus/kernels.mojo:923-1035, :1183-1240).
  */
 size_t heph_attention_ws_bytes(int n_heads, int n_keys);
@@ -93,7 +94,7 @@ int heph_rope_table_bf16(void* table_bf16, int n_pos, int head_dim, double theta
 /*
  * heph_qk_norm_rope_kv on qkv_bf16 into key `pos` of k_cache / v_cache,
  * then heph_attention_fp8kv over pos + 1 keys with the rotated q: the same
- * out, the same cache bytes, in the attention's two launches (the scores
+ * out, the same cache bytes, in the attention's own launches (the scores
  * kernel prepares q and the new key's k and v itself). q in qkv_bf16 is left as it was (not
  * rotated in place). ws: heph_attention_ws_bytes(n_heads, pos + 1) bytes.
  * rope_table: a heph_rope_table_bf16 table of n_rope_pos rows (for this
