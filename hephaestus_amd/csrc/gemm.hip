@@ -198,8 +198,8 @@ __global__ __launch_bounds__(256, 2) void fp8_gemm_kernel(Fp8Operands op)
         }
 }
 
-// Sums the K-split partials of a GEMM in split order, applies per-token and
-// per-channel scales where nothing varied along K ((acc*sa)*sw, the
+// Sums the K-split partials of a GEMM in split order, applies the scales where
+// the partials are unscaled (SCALE: Fp8Operands::scaled_last; (acc*sa)*sw, the
 // association of the unsplit tiles), adds the residual and stores bf16 or f32
 // (four outputs per thread; N % 16 == 0).
 template <bool SCALE>
@@ -240,7 +240,7 @@ hipError_t launch_splitk_reduce(const Fp8Operands& op, hipStream_t stream, const
 {
     const size_t n4 = (size_t)op.M * op.N / 4;
     const int blocks = (int)std::min<size_t>((n4 + 255) / 256, 4096);
-    if (op.s_step == 0)
+    if (op.scaled_last())
         return launch(splitk_reduce_kernel<true>, dim3(blocks), dim3(256), 0, stream, t, op);
     return launch(splitk_reduce_kernel<false>, dim3(blocks), dim3(256), 0, stream, t, op);
 }
@@ -266,7 +266,7 @@ hipError_t launch_big(const Fp8Operands& op, hipStream_t stream, const LaunchTim
     }
     if (op.w_block)
         return launch(fp8_gemm256_kernel<0, BM, BN>, grid, dim3(512), 0, stream, t, op);
-    if (op.s_step == 0)
+    if (op.scaled_last())
         return launch(fp8_gemm256_kernel<2, BM, BN>, grid, dim3(512), 0, stream, t, op);
     return launch(fp8_gemm256_kernel<1, BM, BN>, grid, dim3(512), 0, stream, t, op);
 }
@@ -287,7 +287,7 @@ template <int BM, int BN, int D>
 hipError_t launch_ring(const Fp8Operands& op, hipStream_t stream, const LaunchTiming& t)
 {
     if (op.w_block) return launch_ring_t<kRingBlock, BM, BN, D>(op, stream, t);
-    if (op.s_step == 0) return launch_ring_t<kRingConst, BM, BN, D>(op, stream, t);
+    if (op.scaled_last()) return launch_ring_t<kRingConst, BM, BN, D>(op, stream, t);
     return launch_ring_t<kRingChannel, BM, BN, D>(op, stream, t);
 }
 
@@ -363,8 +363,8 @@ static double ring_estimate(int M, int N, int K, const RingCost& rc, int s)
 // a large tile none: a buffer sized for other rows may be any size); ties go
 // to the earlier tile of kTileCost, then to fewer splits.
 // A forced tile height (gemm_bm) or width (gemm_bn) keeps only the tiles
-// that have it. per_token (nothing varies along K): the large tiles do not
-// split.
+// that have it. per_token (one activation scale a row, with either weight
+// scale): the large tiles do not split.
 // From 33 to 511 rows (per-token scales: to 1023, where the alternative is a
 // large tile over all of K) a ring tile is taken where its estimate is under 0.8 of
 // that: over the 47 shapes of its fit the choice then ran at 0.80 (block
@@ -498,7 +498,7 @@ hipError_t launch_fp8_gemm(const Fp8Operands& op, hipStream_t stream,
     *name = "fp8_gemm_128x128";
     if (op.w_block)
         return launch(fp8_gemm_kernel<0>, dim3(tiles), dim3(256), 0, stream, t, op);
-    if (op.s_step == 0)
+    if (op.scaled_last())
         return launch(fp8_gemm_kernel<2>, dim3(tiles), dim3(256), 0, stream, t, op);
     return launch(fp8_gemm_kernel<1>, dim3(tiles), dim3(256), 0, stream, t, op);
 }

@@ -77,6 +77,12 @@ struct Fp8Operands {
     // carry (unique per launch).
     uint64_t epoch = 0;
     Tuning tune;
+
+    // Whether nothing varies along K (per-channel weights and per-token
+    // activations): the MFMAs then accumulate unscaled, and the epilogue, or
+    // the reduction of a K split's partials, applies (acc*sa)*sw. Block
+    // weights scale every chunk, with per-token activations as well.
+    bool scaled_last() const { return !w_block && s_step == 0; }
 };
 
 hipError_t launch_quant(const uint16_t* x, uint8_t* q, float* scales, int M,
@@ -129,8 +135,9 @@ hipError_t launch_fp8_gemm(const Fp8Operands& op, hipStream_t stream,
 
 // Tile (bm x bn; ring: a tile of gemm_ring.h, else of gemm_big.h) and K
 // splits (1 = none) of the GEMM for M x N x K, splits only where `scratch`
-// bytes hold their partials; forced_bm / forced_bn keep only the large tiles of that height / width (0 =
-// automatic); per_token: per-token and per-channel scales.
+// bytes hold their partials; forced_bm / forced_bn keep only the large
+// tiles of that height / width (0 = automatic); per_token: one activation
+// scale a row.
 struct GemmPlan {
     int bm, bn, splits;
     bool ring;

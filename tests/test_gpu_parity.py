@@ -1426,6 +1426,61 @@ def test_ring_tiles_vs_oracle(tile, M, N, K, mode, out, resid):
     assert np.array_equal(q_ws[: M * K].cpu().numpy().reshape(M, K), qo)
 
 
+# Block weights with per-token activations through the same tiles, and shapes
+# with K splits past the ring's 512 rows of group 128.
+BLOCK_TOKEN_CASES = RING_CASES + [("64x64_splitk", 48, 2560, 9728),
+                                  ("64x32_splitk", 64, 2560, 4096), (None, 300, 2560, 9728),
+                                  (None, 600, 2560, 9728)]
+
+
+@pytest.mark.parametrize("tile,M,N,K", BLOCK_TOKEN_CASES)
+def test_block_weights_per_token_vs_oracle(tile, M, N, K):
+    # The blocks' scales enter chunk by chunk, so a K split's partials are
+    # scaled already and the reduction only sums them. The scratch is the
+    # largest the plan uses; without it (M * K bytes) K is not split: the
+    # sums differ by their f32 rounding.
+    x = O.gen_act_bf16(170 + M, M, K, outlier_p=1e-3)
+    qw, sw = O.gen_weight(171, N, K)
+    r = bf16_of(O.gen_normal(172, M * N).reshape(M, N))
+    q_ws, s_ws = HK.workspace(M, K, group_k=K, n=N)
+    c, q_ws, s_ws = run_linear(qw, sw, x, M=M, N=N, K=K, group_k=K, out=torch.float32, q_ws=q_ws,
+                               s_ws=s_ws)
+    kernel = HK.last_kernel()
+    if tile is not None:
+        assert kernel == "fp8_gemm_" + tile, kernel
+    ref = O.quant_linear(x, qw, sw, group_k=K)
+    got = c.cpu().numpy()
+    assert max_abs_rel(got, ref) <= TOL, (kernel, max_abs_rel(got, ref))
+    base, _, _ = run_linear(qw, sw, x, M=M, N=N, K=K, group_k=K, out=torch.float32)
+    # (a running sum of K / 128 chunks rounds by 2^-24 of it at each, twice)
+    assert max_abs_rel(got, base.cpu().numpy()) <= K // 128 * 2.0 ** -23
+    qo, so = O.quant_act(x, K)
+    assert np.array_equal(q_ws[: M * K].cpu().numpy().reshape(M, K), qo)
+    assert np.array_equal(s_ws[:M].cpu().numpy(), so.reshape(-1))
+    c, _, _ = run_linear(qw, sw, x, M=M, N=N, K=K, group_k=K, residual=dev(r), q_ws=q_ws,
+                         s_ws=s_ws)
+    check_close(host_bf16(c), ref + f32_of_bf16(r), kernel)
+
+
+@pytest.mark.parametrize("tile,M,N,K", BLOCK_TOKEN_CASES)
+def test_block_weights_per_token_exact_integer(tile, M, N, K):
+    # Row scales of 2^-3 .. 2^-1 and block scales of 2^-2 and 2^-1 keep every
+    # partial sum an integer below 2^24 times a power of two: bit for bit.
+    ia, qa = lattice(M, K, 8300 + M)
+    iw, qw = lattice(N, K, 8301)
+    sa = (2.0 ** (np.arange(M) % 3 - 3)).astype(np.float32)
+    nb, kb = -(-N // 128), K // 128
+    sw = (2.0 ** ((np.arange(nb)[:, None] + np.arange(kb)[None, :]) % 2 - 2)).astype(np.float32)
+    iws = iw * np.repeat(np.repeat(sw, 128, 0)[:N], 128, 1)
+    ref = ((ia.astype(np.float64) @ iws.T) * 0.0625 * sa[:, None]).astype(np.float32)
+    q_ws, s_ws = HK.workspace(M, K, group_k=K, n=N)
+    q_ws[: M * K].copy_(dev(qa.reshape(-1)))
+    s_ws.copy_(dev(sa))
+    c, _, _ = run_linear(qw, sw, None, M=M, N=N, K=K, group_k=K, skip_quant=True, q_ws=q_ws,
+                         s_ws=s_ws, out=torch.float32)
+    assert np.array_equal(c.cpu().numpy(), ref), HK.last_kernel()
+
+
 @pytest.mark.parametrize("M,cap", [(73, 128), (96, 128)])
 def test_ring_splits_fit_a_buffer_of_other_rows(M, cap):
     # A workspace sized for 128 rows of down_proj holds fewer partials than the

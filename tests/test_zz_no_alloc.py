@@ -58,3 +58,25 @@ def test_noalloc_matches_linear_two_calls_second_smaller():
     HK.linear_fp8(ref, dev(x), wd, sd, q_ws, s_ws, M, N, K)
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [(48, 2560, 9728), (90, 2560, 4096), (600, 2560, 9728)])
+def test_noalloc_block_weights_per_token(M, N, K):
+    # The fixed array always has split scratch: block weights with per-token
+    # activations against the oracle, and the same bits as heph_fp8_linear with
+    # the scratch it asks for.
+    x = O.gen_act_bf16(70 + M, M, K, outlier_p=1e-3)
+    qw, sw = O.gen_weight(71, N, K)
+    xd, wd, sd = dev(x), dev(qw), dev(sw)
+    got = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda")
+    st = L.lib().heph_fp8_linear_noalloc(
+        got.data_ptr(), L.HEPH_DTYPE_BF16, xd.data_ptr(), wd.data_ptr(), sd.data_ptr(), 128, 128,
+        M, N, K, K, 0, torch.cuda.current_stream().cuda_stream)
+    assert st == L.HEPH_OK, L.strerror(st)
+    ref = torch.zeros_like(got)
+    q_ws, s_ws = HK.workspace(M, K, group_k=K, n=N)
+    HK.linear_fp8(ref, xd, wd, sd, q_ws, s_ws, M, N, K, group_k=K)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+    r = max_abs_rel(f32_of_bf16(host_bf16(got)), O.quant_linear(x, qw, sw, group_k=K))
+    assert r <= 1e-2, (M, r)
