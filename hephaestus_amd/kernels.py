@@ -278,8 +278,9 @@ def linear(c, a, b, m, n, k, ctx=None, *, add_residual=False):
 
 def workspace(m: int, k: int, device="cuda", group_k: int = 128, n: int | None = None):
     """Allocate (a_fp8_ws, act_scale_ws) for up to m rows of width k. With
-    n, a_fp8_ws also holds the scratch the large-M GEMM splits K into for
-    an m x n output (heph_fp8_linear_ws_bytes)."""
+    n, a_fp8_ws also holds the scratch that an m x n output's K splits take
+    (heph_fp8_linear_ws_bytes). A linear may overwrite all of a_fp8_ws past
+    its codes."""
     qb = (L.lib().heph_fp8_linear_ws_bytes(m, n, k) if n is not None
           else L.lib().heph_fp8_q_ws_bytes(m, k))
     q = torch.empty(qb, dtype=torch.uint8, device=device)

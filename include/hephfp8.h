@@ -108,8 +108,15 @@ int heph_fp8_quant_weight(const uint16_t* w_bf16, uint8_t* q, float* scale_inv,
  *   stream               the stream of the reference's DeviceContext
  * On return the workspaces hold x's codes and scales (unless SKIP_QUANT),
  * so later calls on the same x can pass SKIP_QUANT.
- * Past the codes (from the next 256-byte boundary) q_ws is K-split scratch
- * when q_ws_bytes >= heph_fp8_linear_ws_bytes(M, N, K). At M <= 32 the
+ * q_ws_bytes states how much of q_ws is the call's: all of it past the codes
+ * (from the next 256-byte boundary) may be overwritten, with either weight
+ * block and either group_k, for any M. It is the scratch of K splits: a plan
+ * takes as many as it wants and the scratch holds, so the order of an output's
+ * f32 sum (and its last bits) follows q_ws_bytes too. With
+ * heph_fp8_linear_ws_bytes(M, N, K) the whole plan fits (per-token scales may
+ * find room for more); with q_ws_bytes = heph_fp8_q_ws_bytes(M, K) nothing
+ * past the codes is touched and K is not split: pass that where the buffer
+ * holds other data behind them. At M <= 32 the
  * 64-column kernel may sum 2 or 3 K splits inside one launch, where the last
  * split of each column tile waits for the others' completion flags for a
  * bounded time (~0.3 s). If a wait ever gives up, that tile's outputs are
@@ -252,12 +259,13 @@ size_t heph_fp8_s_ws_floats(int M, int K, int group_k);
 
 /*
  * Optional larger q_ws for (M, N, K): the activation codes, rounded up to
- * 256 bytes, plus scratch for the fp32 partials of the large-M GEMM when it
- * splits K (M >= 128 and few output tiles, e.g. M = 512 with N = 2560).
- * Passing a q_ws of this size (q_ws_bytes) lets heph_fp8_linear use the
- * part past the codes as that scratch; with the minimal q_ws it does not
- * split. No counterpart in the reference, whose workspaces are sized for
- * the codes and scales only (forward.mojo:121-125).
+ * 256 bytes, plus the scratch that heph_fp8_linear's plan for block weights
+ * splits K into (fp32 partials; from M = 25 on, where few output tiles or a
+ * long K leave compute units idle, e.g. M = 48 or 512 with N = 2560). It does
+ * not grow steadily with M: a buffer sized for the largest M may hold fewer
+ * splits of a smaller one, which then takes those (M > 32) or none. With the
+ * minimal q_ws nothing is split. No counterpart in the reference, whose
+ * workspaces are sized for the codes and scales only (forward.mojo:121-125).
  */
 size_t heph_fp8_linear_ws_bytes(int M, int N, int K);
 

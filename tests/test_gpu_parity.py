@@ -1503,6 +1503,27 @@ def test_ring_splits_fit_a_buffer_of_other_rows(M, cap):
     assert bool((buf[need:] == 0xA5).all())
 
 
+@pytest.mark.parametrize("M,N,K,mode", [(45, 1776, 2192, "channel_token")] + [
+    (*shape, mode) for shape in ((28, 19456, 2560), (48, 2560, 9728), (333, 2560, 4096),
+                                 (512, 2560, 9728))
+    for mode in ("block", "block_token", "channel_token", "channel_g128")])
+def test_q_ws_bytes_bounds_the_scratch(M, N, K, mode):
+    # q_ws_bytes is how much of the buffer is the call's: with the codes' own
+    # size what follows them stays as it was (and K is not split), with the size
+    # of the split plan what follows that.
+    qw, sw = O.gen_weight(180, N, K) if mode.startswith("block") else \
+        O.quant_weight(O.gen_normal(180, N * K, 0.0, 0.02).reshape(N, K), 1, K)
+    g = K if mode.endswith("token") else 128
+    x = O.gen_act_bf16(181 + M, M, K)
+    for need in (L.lib().heph_fp8_q_ws_bytes(M, K), L.lib().heph_fp8_linear_ws_bytes(M, N, K)):
+        buf = torch.full((need + 65536,), 0xA5, dtype=torch.uint8, device="cuda")
+        s_ws = torch.zeros(M * (K // g), dtype=torch.float32, device="cuda")
+        run_linear(qw, sw, x, M=M, N=N, K=K, group_k=g, q_ws=buf[:need], s_ws=s_ws)
+        assert bool((buf[need:] == 0xA5).all())
+        if need == M * K:
+            assert not HK.last_kernel().endswith("_splitk"), HK.last_kernel()
+
+
 @pytest.mark.parametrize("tile,M,N,K", RING_CASES)
 def test_ring_tiles_exact_integer(tile, M, N, K):
     # Every partial sum is an integer below 2^24 times a power of two: bit for
