@@ -90,12 +90,12 @@ using ic = std::integral_constant<int, V>;
 
 // The chunk-start wait of the large-M kernel: the wave's LDS reads and
 // scalar loads done (lgkmcnt(0)) and all its vector memory instructions
-// but the newest n (vmcnt(n), n = 9, 8, 4 or 0: with three stages the DMA
-// of the next chunk may stay in flight).
+// but the newest n (vmcnt(n): with three stages the DMA of the next chunk,
+// 3 to 10 instructions of this wave, may stay in flight; any other n waits
+// for all).
 __device__ __forceinline__ void wait_stage(int n)
 {
     switch (n) {
-    case 11: __builtin_amdgcn_s_waitcnt(0x007B); break;
     case 10: __builtin_amdgcn_s_waitcnt(0x007A); break;
     case 9: __builtin_amdgcn_s_waitcnt(0x0079); break;
     case 8: __builtin_amdgcn_s_waitcnt(0x0078); break;
@@ -104,7 +104,6 @@ __device__ __forceinline__ void wait_stage(int n)
     case 5: __builtin_amdgcn_s_waitcnt(0x0075); break;
     case 4: __builtin_amdgcn_s_waitcnt(0x0074); break;
     case 3: __builtin_amdgcn_s_waitcnt(0x0073); break;
-    case 2: __builtin_amdgcn_s_waitcnt(0x0072); break;
     default: __builtin_amdgcn_s_waitcnt(0x0070); break;
     }
     asm volatile("" ::: "memory");
@@ -347,10 +346,13 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm256_kernel(Fp8Operands op)
     // over the 2 row tiles of BM = 64, so that every part goes out)
     constexpr int kPer = L_MT >= 8 ? 2 : L_MT >= 4 ? 3 : (kParts + L_MT - 1) / L_MT;
     static_assert(kPer * L_MT >= kParts, "every DMA part is issued");
+    // A wave's A parts are all inside the tile or all outside it: one test a
+    // chunk instead of one a part
+    constexpr bool kWholeWaves = L_BM % (8 * NAP) == 0;
     auto issue_part = [&](int ja, int jw, auto abufc, int bbuf, int part) {
         constexpr int abuf = decltype(abufc)::value;
         if (part < NAP) {
-            if ((wave * NAP + part) * 8 < L_BM)
+            if (kWholeWaves ? wave * NAP * 8 < L_BM : (wave * NAP + part) * 8 < L_BM)
                 dma16(rq, aoff[part], (uint32_t)ja * kChunk,
                       smem + T::a_at(abuf) + (wave * NAP + part) * 8 * kChunk);
         } else if (part == kScalePart) {
@@ -425,7 +427,9 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm256_kernel(Fp8Operands op)
     };
 
     // DMA instructions a wave issues per chunk (A rows, B rows, row scales).
-    const int n_parts = max(0, min(NAP, L_BM / 8 - wave * NAP)) + NBP + (RESCALE && wave * 64 < L_BM ? 1 : 0);
+    const int a_parts = kWholeWaves ? (wave * NAP * 8 < L_BM ? NAP : 0)
+                                    : max(0, min(NAP, L_BM / 8 - wave * NAP));
+    const int n_parts = a_parts + NBP + (RESCALE && wave * 64 < L_BM ? 1 : 0);
 
     // One 128-wide chunk j held in A stage buf (a compile-time constant)
     // and B stage bst. The wave's nine DMA instructions (A rows and scales
