@@ -7,7 +7,7 @@
 // kernel in bf16_skinny.hip.
 //
 // The DMA-staged tiles of gemm_big.h and gemm_ring.h in their bf16 form take
-// every call whose operands' byte offsets fit 32 bits: no per-chunk scales,
+// most calls whose operands' byte offsets fit 32 bits: no per-chunk scales,
 // so the MFMAs accumulate in place. They are bound by the weight stream (up
 // to M of about 100) or by the MFMAs; what costs beside that is rows of the
 // last tile past M, a last round of tiles that leaves CUs idle, and the DMA's
@@ -18,7 +18,8 @@
 // 390; 4096 x 6144 x 2560 181 -> 119; M = 45 at 4256 x 1408 21.8 -> 11.0; over
 // 51 shapes (M 33 .. 4096) 0.50 to 0.996 of its time, 0.70 in the mean.
 //
-// The register-staged kernel, for larger operands:
+// The register-staged kernel, for larger operands and where its two tiles on a
+// CU beat the ring tiles (bf16_gemm_tile):
 //   * 128 x 128 output tile per 256-thread workgroup, 2 x 2 waves of
 //     64 x 64, each wave 4 x 4 v_mfma_f32_16x16x32_bf16 per 32-wide K step,
 //     two steps per 64-element (128-byte) chunk; the MFMAs accumulate in
@@ -168,17 +169,17 @@ namespace {
 // Tiles of the DMA-staged kernels and the model that picks one: with n tiles
 // on the fullest CU and KC chunks of 64 elements, n g + KC max(c1, n c) + 2 us,
 // but at least the weights and the output at 5 TB/s, the rate the tiles reach
-// where the stream bounds them; ties go to the earlier entry. c1 is a chunk's
-// latency with one workgroup on the CU, c its share of the CU, g a tile's
-// prologue and epilogue; fitted to MI355X times at 51 shapes (M 33 .. 4096,
-// N 4096 .. 151936, K 1024 .. 2560), over which the choice is on average 3 %
-// slower than the fastest tile.
+// where the stream bounds them; ties go to the earlier entry. c1 is a chunk's latency with one workgroup on the CU, c its share of the CU,
+// g a tile's prologue and epilogue; fitted to MI355X times at 51 shapes (M 33 ..
+// 4096, N 4096 .. 151936, K 1024 .. 2560), over which the choice is on average
+// 3 % slower than the fastest tile. (The coefficients are the fit's, not a
+// tile's latencies one by one.)
 struct Bf16Tile {
     int bm, bn;
     double g, c1, c;
     const char* name;
 };
-enum { kT160x320, kT160x256, kT128x256, kT256x256, kT288x192, kT128x128, kT64x64 };
+enum { kT160x320, kT160x256, kT128x256, kT256x256, kT288x192, kT128x128, kT64x64, kReg };
 constexpr Bf16Tile kBf16Tiles[] = {
     {160, 320, 4.08, 0.109, 1.341, "bf16_gemm_160x320"},
     {160, 256, 3.53, 1.003, 1.159, "bf16_gemm_160x256"},
@@ -194,6 +195,21 @@ constexpr Bf16Tile kBf16Tiles[] = {
 // The 128- to 288-row tiles of gemm_big.h from M = 65 on (up to 64 rows they
 // would be at most half full); outputs narrower than 4096 columns, where the
 // fit has no shapes, keep the 128 x 128 tile.
+// A CU holds two 128 x 128 workgroups of the register-staged kernel, but one
+// of the ring's 128 x 128 or two of its 64 x 64. Where the model takes a ring
+// tile and there are more than 256 tiles of 128 x 128, the register-staged
+// kernel is therefore the faster one for short rows (M > 64, K <= 384: one
+// workgroup's stores hide the other's prologue), and up to 64 rows where its
+// rounds are more than 65 % full and either K <= 2048 or all of it fits one
+// round. MI355X, register-staged against the ring tile: 2528 x 1552 x 128 7.0
+// and 10.0 us, 56 x 59312 x 128 8.8 and 11.9, 65 x 87392 x 256 17.8 and 22.3,
+// 59 x 62000 x 512 17.9 and 21.0, 62 x 52624 x 2560 62.1 and 67.8; on the other
+// side 39 x 80656 x 2048 (rounds 62 % full) 97.5 and 74.3, 64 x 151936 x 2560
+// 189 and 176, 3893 x 816 x 512 12.3 and 10.0. Over 838 drawn shapes (M 33 ..
+// 4096, N 16 .. 152000, K 128 .. 8192) the choice takes 0.78 of the
+// register-staged kernel's time; 20 of them take more than 1.03 (1.15 at worst),
+// 18 with K <= 640 on the tiles of 128 rows and more, which take 0.84 of its
+// time there in the mean.
 int bf16_gemm_tile(int M, int N, int K, bool c_f32)
 {
     const double floor_us =
@@ -212,6 +228,12 @@ int bf16_gemm_tile(int M, int N, int K, bool c_f32)
             best = i;
         }
     }
+    const long regs = (long)((M + 127) / 128) * ((N + 127) / 128);
+    if (best >= kT128x128 && regs > kPlanCUs) {
+        const long slots = 2 * kPlanCUs, rounds = (regs + slots - 1) / slots;
+        const bool full = 100 * regs > 65 * rounds * slots;
+        if (M > 64 ? K <= 384 : full && (K <= 2048 || rounds == 1)) return kReg;
+    }
     return best;
 }
 
@@ -219,7 +241,9 @@ hipError_t launch_bf16_gemm(void* c, bool c_f32, bool residual, const uint16_t* 
                             const uint16_t* w, int M, int N, int K, hipStream_t stream,
                             const LaunchTiming& t, const char** name)
 {
-    if ((long)M * K < (1L << 30) && (long)N * K < (1L << 30)) {
+    const bool small_offsets = (long)M * K < (1L << 30) && (long)N * K < (1L << 30);
+    const int i = small_offsets ? bf16_gemm_tile(M, N, K, c_f32) : kReg;
+    if (i != kReg) {
         Fp8Operands op{};
         op.x = x;
         op.w = reinterpret_cast<const uint8_t*>(w);
@@ -229,7 +253,6 @@ hipError_t launch_bf16_gemm(void* c, bool c_f32, bool residual, const uint16_t* 
         op.M = M;
         op.N = N;
         op.K = K;
-        const int i = bf16_gemm_tile(M, N, K, c_f32);
         const Bf16Tile& b = kBf16Tiles[i];
         const dim3 grid(((M + b.bm - 1) / b.bm) * ((N + b.bn - 1) / b.bn));
         *name = b.name;
@@ -246,7 +269,7 @@ hipError_t launch_bf16_gemm(void* c, bool c_f32, bool residual, const uint16_t* 
     const Bf16GemmArgs a{c, x, w, M, N, K, c_f32, residual};
     const long tiles = (long)((M + kGbM - 1) / kGbM) * ((N + kGbN - 1) / kGbN);
     if (tiles > 0x7fffffffL) return hipErrorInvalidValue;
-    *name = "bf16_gemm_128x128";
+    *name = "bf16_gemm_128x128_reg";
     return launch(bf16_gemm_kernel, dim3((unsigned)tiles), dim3(256), 0, stream, t, a);
 }
 

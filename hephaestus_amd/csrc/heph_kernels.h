@@ -179,8 +179,10 @@ hipError_t launch_fp8_gemv_wide(const Fp8Operands& op, hipStream_t stream,
 void gemv_wide_shape(int M, int N, int K, const Tuning& tune, int* tiles, int* waves, int* u);
 bool gemv_wide_routes(int M, int N, int K, bool codes);
 
-// bf16 x [M,K] @ w [N,K]^T, f32 accumulation, M > 32 (bf16_gemm.hip):
-// 128x128 tiles; the residual is the output buffer's contents.
+// bf16 x [M,K] @ w [N,K]^T, f32 accumulation, M > 32 (bf16_gemm.hip: the
+// bf16 form of gemm_big.h's and gemm_ring.h's tiles, or the register-staged
+// kernel these arguments are for); the residual is the output buffer's
+// contents.
 struct Bf16GemmArgs {
     void* c;
     const uint16_t* x;

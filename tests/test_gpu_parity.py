@@ -725,6 +725,52 @@ def test_bf16_gemm_every_tile(M, N, K, tile, out, resid):
         assert bad.size == 0, (bad.size, bad[:5])
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (33, 42640, 128), (64, 42752, 640),        # one round of its tiles, two thirds full
+    (35, 109328, 384),                         # two rounds
+    (70, 35296, 128), (2177, 1936, 384)])      # short rows, more than 256 tiles
+@pytest.mark.parametrize("out,resid", [("f32", False), ("bf16", True)])
+def test_bf16_gemm_register_staged(M, N, K, out, resid):
+    # The register-staged kernel where the choice of tile takes it (ragged last
+    # row and column tiles); bounds as test_bf16_gemm.
+    x = O.gen_act_bf16(160 + M, M, K)
+    w = bf16_of(O.gen_normal(161 + N, N * K, 0.0, 0.02)).reshape(N, K)
+    dt = torch.float32 if out == "f32" else torch.bfloat16
+    res = bf16_of(O.gen_normal(163 + M, M * N, 0.0, 1.0)).reshape(M, N)
+    c = dev(res) if resid else torch.zeros(M, N, dtype=dt, device="cuda")
+    HK.linear(c, dev(x), dev(w), M, N, K, add_residual=resid)
+    torch.cuda.synchronize()
+    assert HK.last_kernel() == "bf16_gemm_128x128_reg", HK.last_kernel()
+    want = O.bf16_linear(x, w) + (f32_of_bf16(res).astype(np.float64) if resid else 0.0)
+    if out == "f32":
+        assert max_abs_rel(c.cpu().numpy(), want) < 1e-5
+    else:
+        err = np.abs(f32_of_bf16(host_bf16(c)).astype(np.float64) - want)
+        assert np.all(err <= 2.0 ** -8 * np.abs(want) + 1e-5 * np.abs(want).max())
+
+
+def test_bf16_gemm_past_32_bit_offsets():
+    # N * K of more than 2^30 elements: the register-staged kernel, against the
+    # DMA-staged tiles on pieces of the same weight (the chunks are summed in
+    # one order: equal bit for bit) and float64 on the last columns.
+    M, K = 33, 2048
+    N = 2 ** 19 + 16
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    w = torch.empty(N, K, dtype=torch.bfloat16, device="cuda").normal_(0.0, 0.02)
+    c = torch.zeros(M, N, dtype=torch.float32, device="cuda")
+    HK.linear(c, x, w, M, N, K)
+    torch.cuda.synchronize()
+    assert HK.last_kernel() == "bf16_gemm_128x128_reg", HK.last_kernel()
+    for n0 in (0, N // 2, N - 4112):
+        p = torch.zeros(M, 4112, dtype=torch.float32, device="cuda")
+        HK.linear(p, x, w[n0: n0 + 4112], M, 4112, K)
+        torch.cuda.synchronize()
+        assert HK.last_kernel() == "bf16_gemm_64x64", HK.last_kernel()
+        assert torch.equal(c[:, n0: n0 + 4112], p), n0
+    ref = x.double() @ w[-64:].double().T
+    assert float((c[:, -64:].double() - ref).abs().max() / ref.abs().max()) < 1e-5
+
+
 def test_bf16_gemm_lm_head_rows():
     # The lm_head (151936 x 2560) over 64 positions: 8 sampled rows against
     # the oracle (rows of C are independent), greedy argmax agreeing.
