@@ -169,7 +169,11 @@ namespace {
 // Tiles of the DMA-staged kernels and the model that picks one: with n tiles
 // on the fullest CU and KC chunks of 64 elements, n g + KC max(c1, n c) + 2 us,
 // but at least the weights and the output at 5 TB/s, the rate the tiles reach
-// where the stream bounds them; ties go to the earlier entry. c1 is a chunk's latency with one workgroup on the CU, c its share of the CU,
+// where the stream bounds them. Of two tiles at that bound the one with less
+// time of its own is taken among the first three (a call it bounds has few
+// rows), else the earlier entry (92 x 119680 x 2304 on 160 x 320 136 us, on the
+// register-staged kernel 129; 108 x 127808 x 1408 95.1, on 128 x 256 90.6).
+// c1 is a chunk's latency with one workgroup on the CU, c its share of the CU,
 // g a tile's prologue and epilogue; fitted to MI355X times at 51 shapes (M 33 ..
 // 4096, N 4096 .. 151936, K 1024 .. 2560), over which the choice is on average
 // 3 % slower than the fastest tile. (The coefficients are the fit's, not a
@@ -206,24 +210,27 @@ constexpr Bf16Tile kBf16Tiles[] = {
 // 59 x 62000 x 512 17.9 and 21.0, 62 x 52624 x 2560 62.1 and 67.8; on the other
 // side 39 x 80656 x 2048 (rounds 62 % full) 97.5 and 74.3, 64 x 151936 x 2560
 // 189 and 176, 3893 x 816 x 512 12.3 and 10.0. Over 838 drawn shapes (M 33 ..
-// 4096, N 16 .. 152000, K 128 .. 8192) the choice takes 0.78 of the
-// register-staged kernel's time; 20 of them take more than 1.03 (1.15 at worst),
-// 18 with K <= 640 on the tiles of 128 rows and more, which take 0.84 of its
-// time there in the mean.
+// 4096, N 16 .. 152000, K 128 .. 8192) the choice takes 0.77 of the
+// register-staged kernel's time; 9 of them take more than 1.03 (1.10 at worst),
+// 7 with K <= 640 on the tiles of 128 rows and more, which take 0.82 of its
+// time there in the mean. (Of 750 shapes drawn afterwards one takes more, 1.07.)
 int bf16_gemm_tile(int M, int N, int K, bool c_f32)
 {
     const double floor_us =
         3.0 + (2.0 * N * K + (double)M * N * (c_f32 ? 4 : 2)) / 5.0e6;
     int best = kT128x128;
-    double best_t = -1.0;
+    double best_t = -1.0, best_own = 0.0;
     for (int i = 0; i <= kT64x64; ++i) {
         const Bf16Tile& t = kBf16Tiles[i];
         if (N < 4096 && i != kT128x128) continue;
         if (M <= 64 && i < kT128x128) continue;
         const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         const double n = (double)((tiles + kPlanCUs - 1) / kPlanCUs), kc = K / 64;
-        const double us = std::max(floor_us, 2.0 + n * t.g + kc * std::max(t.c1, n * t.c));
-        if (best_t < 0.0 || us < best_t) {
+        const double own = 2.0 + n * t.g + kc * std::max(t.c1, n * t.c);
+        const double us = std::max(floor_us, own);
+        if (best_t < 0.0 || us < best_t ||
+            (us == best_t && i <= kT128x256 && own < best_own)) {
+            best_own = own;
             best_t = us;
             best = i;
         }

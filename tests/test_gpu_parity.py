@@ -749,6 +749,13 @@ def test_bf16_gemm_register_staged(M, N, K, out, resid):
         assert np.all(err <= 2.0 ** -8 * np.abs(want) + 1e-5 * np.abs(want).max())
 
 
+@pytest.mark.parametrize("M,N,K,tile", [(65, 46480, 256, "128x256"), (130, 40976, 256, "160x256")])
+def test_bf16_gemm_stream_bound_tile(M, N, K, tile):
+    # Several tiles at the weight stream's bound: the one with least time of its
+    # own among the 256- and 320-column ones, not the first.
+    test_bf16_gemm_every_tile(M, N, K, tile, "f32", False)
+
+
 def test_bf16_gemm_past_32_bit_offsets():
     # N * K of more than 2^30 elements: the register-staged kernel, against the
     # DMA-staged tiles on pieces of the same weight (the chunks are summed in
