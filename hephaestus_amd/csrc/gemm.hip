@@ -366,12 +366,15 @@ static double ring_estimate(int M, int N, int K, const RingCost& rc, int s)
 // that have it. per_token (one activation scale a row, with either weight
 // scale): the large tiles do not split.
 // From 33 to 511 rows (per-token scales: to 1023, where the alternative is a
-// large tile over all of K) a ring tile is taken where its estimate is under 0.8 of
-// that: over the 47 shapes of its fit the choice then ran at 0.80 (block
-// scales) and 0.69 (per-token) of the large tiles' time, 1.02 at worst (0.8 to
-// 1.0: up to 1.19; from M = 470 on the two run alike). Past K = 4096 the ring
-// splits first: one workgroup's chain of chunks is then longer than a
-// reduction.
+// large tile over all of K) a ring tile is taken where its estimate is under
+// 0.8 of that, or under 0.7 where the large tile would split a K past 4608. Of
+// 1494 drawn calls (M 33 .. 1100, N 16 .. 19456, K 128 .. 16384, every scale
+// format, workspaces of several sizes) that a line of 0.8 gave a ring tile, those
+// under 0.7 ran at 0.72 of the large tile's time; from 0.7 to 0.8 they ran at
+// 0.84 against an unsplit large tile (0.98 at worst), at 1.00 against a split
+// one (0.80 to 1.13; 13 of the 14 past 1.015 with K of 4736 and more). Past
+// K = 4096 the ring splits first: one workgroup's chain of chunks is then longer
+// than a reduction.
 GemmPlan gemm_plan(int M, int N, int K, size_t scratch, int forced_bm, int forced_bn,
                    bool per_token)
 {
@@ -405,7 +408,7 @@ GemmPlan gemm_plan(int M, int N, int K, size_t scratch, int forced_bm, int force
     if (!fits(best.splits)) large(1);
     if (best.bm == 0) best = GemmPlan{forced_bm >= 64 ? forced_bm : 256, 256, 1, false};
     if (M <= 32 || M >= (per_token ? 1024 : 512) || forced_bm || forced_bn) return best;
-    best_t *= 0.8;
+    best_t *= best.splits > 1 && K > 4608 ? 0.7 : 0.8;
     const auto ring = [&](int s0, int s1) {
         for (const auto& rc : kRingCost) {
             for (int s = s0; s <= s1 && fits(s); ++s) {

@@ -1479,6 +1479,24 @@ def test_ring_tiles_vs_oracle(tile, M, N, K, mode, out, resid):
     assert np.array_equal(q_ws[: M * K].cpu().numpy().reshape(M, K), qo)
 
 
+@pytest.mark.parametrize("tile,M,N,K", [("64x192_splitk", 320, 1232, 8448),
+                                        ("64x192_splitk", 386, 608, 14080),
+                                        ("64x256_splitk", 73, 4624, 9600)])
+def test_long_k_stays_on_split_large_tiles(tile, M, N, K):
+    # Past K = 4608 a large tile's K splits are left to a ring tile's only where
+    # those are estimated well under them: exact sums on either, bit for bit.
+    ia, qa = lattice(M, K, 8400 + M)
+    iw, qw = lattice(N, K, 8401)
+    ref = ((ia.astype(np.float64) @ iw.astype(np.float64).T) * 0.0625 * 2.0 ** -5)
+    q_ws, s_ws = HK.workspace(M, K, n=N)
+    q_ws[: M * K].copy_(dev(qa.reshape(-1)))
+    s_ws.fill_(2.0 ** -3)
+    c, _, _ = run_linear(qw, np.full((-(-N // 128), K // 128), 2.0 ** -2, np.float32), None, M=M,
+                         N=N, K=K, skip_quant=True, q_ws=q_ws, s_ws=s_ws)
+    assert HK.last_kernel() == "fp8_gemm_" + tile, HK.last_kernel()
+    assert np.array_equal(host_bf16(c), bf16_of(ref.astype(np.float32)))
+
+
 # Block weights with per-token activations through the same tiles, and shapes
 # with K splits past the ring's 512 rows of group 128.
 BLOCK_TOKEN_CASES = RING_CASES + [("64x64_splitk", 48, 2560, 9728),
