@@ -269,9 +269,10 @@ constexpr int kAttnSplit = 256;
 template <int G>
 constexpr int kAttnKPT = G == 8 ? 4 : 2;
 // Scores workgroups that MI355X holds at once: two 1024-thread ones on each of
-// its 256 CUs with one query head (54 registers), else one.
-template <int G>
-constexpr int kAttnSlots = (G == 1 ? 2 : 1) * kPlanCUs;
+// its 256 CUs up to 64 registers, else one. The looped form has 48 registers with
+// one query head and 66 and more beyond, the other 60 with two query heads.
+template <int G, bool LOOP>
+constexpr int kAttnSlots = (G == 1 || (G == 2 && !LOOP) ? 2 : 1) * kPlanCUs;
 
 // The workspace holds the scores [n_heads][n_keys] (fp32).
 
@@ -325,7 +326,7 @@ struct QkvPrep {
 //
 // LOOP: a workgroup takes every `stride`-th split from its first on, loading the
 // next split's rows before it scores the current one: with more splits than
-// workgroups fit the device (kAttnSlots), each prepares its q heads once and no
+// workgroups fit the device (launch_attention), each prepares its q heads once and no
 // second round of workgroups starts behind the first (the attention at 8 kv x 4
 // query heads, graph-replayed: 8193 keys 19.7 -> 18.4 us, 40000 59.3 -> 53.8).
 template <int G, bool QKV, int KPT, bool LOOP>
@@ -804,18 +805,30 @@ hipError_t launch_attention(uint16_t* out, const uint16_t* q, const uint8_t* kc,
                             const QkvPrep& prep = QkvPrep{})
 {
     const int splits = (n_keys + kAttnSplit - 1) / kAttnSplit;
-    const int per_kv = std::max(1, kAttnSlots<G> / n_kv);    // workgroups that fit at once
-    constexpr int NT = 8 * kAttnSplit / kAttnKPT<G>;
-    const int stride = std::min(splits, per_kv), blocks = n_kv * stride;
+    // The looped form, a kv head's splits over the workgroups that fit at once,
+    // where they do not all fit. Without q heads to prepare it saves only the
+    // rounds behind the first, so it has to need no more turns than the other
+    // form rounds, which with two query heads holds twice the workgroups, and
+    // where n_kv does not divide the slots fills those the loop leaves idle
+    // (kv heads x query heads, keys: 16 x 2, 8676 19.3 us in rounds, 20.2 looped;
+    // 160 x 2, 8000 152 and 163; 300 x 1, 6000 147 and 160; with the q heads
+    // 160 x 2 187 and 166, 300 x 1 193 and 161).
+    const int per_kv = std::max(1, kAttnSlots<G, true> / n_kv);    // that fit at once
+    constexpr int NT = 8 * kAttnSplit / kAttnKPT<G>, ONCE = kAttnSlots<G, false>;
+    const int turns = (splits + per_kv - 1) / per_kv *
+                      ((n_kv * per_kv + kAttnSlots<G, true> - 1) / kAttnSlots<G, true>);
+    const int rounds = (int)(((long)splits * n_kv + ONCE - 1) / ONCE);
+    const bool looped = splits > per_kv && (prep.qkv || turns <= rounds);
+    const int stride = looped ? per_kv : splits, blocks = n_kv * stride;
     auto scores = [&](auto qkv, auto loop) {
         attn_scores_kernel<G, decltype(qkv)::value, kAttnKPT<G>, decltype(loop)::value>
             <<<blocks, NT, 0, s>>>(ws, q, kc, kv_scale, n_kv, n_keys, splits, stride, prep);
     };
     if (prep.qkv) {
-        if (splits > per_kv) scores(std::true_type{}, std::true_type{});
+        if (looped) scores(std::true_type{}, std::true_type{});
         else scores(std::true_type{}, std::false_type{});
     } else {
-        if (splits > per_kv) scores(std::false_type{}, std::true_type{});
+        if (looped) scores(std::false_type{}, std::true_type{});
         else scores(std::false_type{}, std::false_type{});
     }
     const dim3 vgrid(n_kv * G * 8);

@@ -252,6 +252,16 @@ def test_attention_qkv_long_matches_separate_ops(nh, nkv, pos):
     test_attention_qkv_matches_separate_ops(pos, nh, nkv)
 
 
+@pytest.mark.parametrize("nh,nkv,n", [(520, 520, 700), (320, 160, 600), (600, 300, 464),
+                                      (160, 160, 1100)],
+                         ids=["rounds-g1", "rounds-g2", "rounds-g2-many", "looped-g1"])
+def test_attention_kv_heads_that_do_not_divide_the_slots(nh, nkv, n):
+    # More splits than workgroups fit at once: in rounds where the looped form
+    # would need more turns, looped with the q heads to prepare in any case.
+    test_attention_gqa_vs_oracle(nh, nkv, n)
+    test_attention_qkv_matches_separate_ops(n - 1, nh, nkv)
+
+
 def test_attention_rejects_long_context_and_small_workspace():
     z = torch.zeros(16, dtype=torch.uint8, device="cuda")
     with pytest.raises(HephError):
