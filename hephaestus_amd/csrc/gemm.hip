@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(Fp8Operands op)
         if constexpr (SCALE) {
             const size_t row = i * 4 / op.N;
             const float sa = op.s[row];
-            const f32x4 sw = *reinterpret_cast<const f32x4*>(op.sw + (i * 4 - row * op.N));
+            const f32x4 sw = ldf4(op.sw + (i * 4 - row * op.N));
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = (v[e] * sa) * sw[e];
         }

@@ -294,7 +294,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(
             }
             if constexpr (SM == kRingConst) {
                 // the reference's association (wmma_gfx12.mojo:711-712, :848)
-                const f32x4 sw = *reinterpret_cast<const f32x4*>(op.sw + col);
+                const f32x4 sw = ldf4(op.sw + col);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     v[e] = M == 1 ? v[e] * (sa * sw[e]) : (v[e] * sa) * sw[e];

@@ -333,4 +333,12 @@ __device__ __forceinline__ uint4 ldg16u(const void* p)
     return *reinterpret_cast<const uint4*>(p);
 }
 
+// Four consecutive floats at any float's address (weight scales need no more
+// than that: a caller may pass a slice); one 16-byte load here too.
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+__device__ __forceinline__ f32x4 ldf4(const float* p)
+{
+    return *reinterpret_cast<const f32x4_a4*>(p);
+}
+
 }  // namespace heph

@@ -1552,6 +1552,28 @@ def test_block_weights_per_token_exact_integer(tile, M, N, K):
     assert np.array_equal(c.cpu().numpy(), ref), HK.last_kernel()
 
 
+@pytest.mark.parametrize("M,N,K", [(147, 1504, 640), (45, 1776, 4224)])
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_channel_scales_at_any_float_address(M, N, K, off):
+    # Per-channel scales that start between 16-byte boundaries (a slice of a
+    # larger array), unsplit and split over K: the bits of aligned ones.
+    x = dev(O.gen_act_bf16(190 + M, M, K))
+    qw, sw = O.quant_weight(O.gen_normal(191, N * K, 0.0, 0.02).reshape(N, K), 1, K)
+    w, outs = dev(qw), []
+    buf = torch.zeros(N + 4, dtype=torch.float32, device="cuda")
+    for o in (0, off):
+        s = buf[o: o + N]
+        s.copy_(dev(sw.reshape(-1)))
+        assert s.data_ptr() % 16 == 4 * o
+        q_ws, s_ws = HK.workspace(M, K, group_k=K, n=N)
+        c = torch.zeros(M, N, dtype=torch.float32, device="cuda")
+        HK.linear_fp8(c, x, w, s, q_ws, s_ws, M, N, K, group_k=K)
+        torch.cuda.synchronize()
+        outs.append(c)
+        assert HK.last_kernel().endswith("_splitk") == (K > 4096), HK.last_kernel()
+    assert torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("M,cap", [(73, 128), (96, 128)])
 def test_ring_splits_fit_a_buffer_of_other_rows(M, cap):
     # A workspace sized for 128 rows of down_proj holds fewer partials than the
