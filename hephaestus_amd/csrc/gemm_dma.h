@@ -63,9 +63,8 @@ typedef const __attribute__((address_space(4))) float* const_f32_ptr;
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
-// Two floats -> two bf16 (round to nearest even) in one v_cvt_pk_bf16_f32;
-// equal bit for bit to f32_to_bf16 on non-NaN values (checked on the GPU
-// against the f32 output of the same kernel rounded on the host).
+// Two floats -> two bf16 (round to nearest even) in one v_cvt_pk_bf16_f32,
+// each as f32_to_bf16 rounds it.
 __device__ __forceinline__ uint32_t pack_bf16_hw(float a, float b)
 {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));

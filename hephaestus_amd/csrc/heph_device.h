@@ -65,9 +65,9 @@ __device__ __forceinline__ float bf16lo(uint32_t u) { return __uint_as_float(u <
 __device__ __forceinline__ float bf16hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
 
 // f32 -> bf16 bits, round to nearest even, a NaN quieted with its sign and
-// upper payload kept: v_cvt_pk_bf16_f32, equal for all 2^32 inputs to the
-// integer form (add 0x7fff plus the lowest kept bit, shift; NaN: or 0x40),
-// which costs six instructions.
+// upper payload kept: v_cvt_pk_bf16_f32, equal for all 2^32 inputs (the tests
+// compare them) to the integer form (add 0x7fff plus the lowest kept bit,
+// shift; NaN: or 0x40), which costs six instructions.
 __device__ __forceinline__ uint16_t f32_to_bf16(float f)
 {
     return __builtin_bit_cast(uint16_t, (__bf16)f);

@@ -1574,6 +1574,32 @@ def test_channel_scales_at_any_float_address(M, N, K, off):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("M", [1, 33])
+def test_bf16_rounding_of_every_f32(M):
+    # All 2^32 f32 values through the outputs' rounding (per-channel scales of a
+    # product that is exactly 1), one output and pairs of them: the integer form of
+    # round to nearest even, a NaN quieted with its sign and upper payload.
+    N, K, step = 1 << 20, 256, 1 << 20
+    w = torch.zeros(N, K, dtype=torch.uint8, device="cuda")
+    w[:, 0] = 0x38                                                    # 1.0
+    q_ws = torch.zeros(M * K, dtype=torch.uint8, device="cuda")
+    q_ws[::K] = 0x38
+    s_ws = torch.ones(M, dtype=torch.float32, device="cuda")
+    c = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda")
+    base = torch.arange(step, dtype=torch.int32, device="cuda")
+    bad = torch.zeros((), dtype=torch.int64, device="cuda")
+    for i in range((1 << 32) // step):
+        u = base + ((i * step + (1 << 31)) % (1 << 32) - (1 << 31))
+        HK.linear_fp8(c, None, w, u.view(torch.float32), q_ws, s_ws, M, N, K, do_quantize=False,
+                      group_k=K)
+        r = (u + 0x7fff + ((u >> 16) & 1)) >> 16
+        nan = (u & 0x7fffffff) > 0x7f800000
+        want = torch.where(nan, (u >> 16) | 0x40, r).to(torch.int16)
+        bad += (c[0].view(torch.int16) != want).sum() + (c[M - 1].view(torch.int16) != want).sum()
+    torch.cuda.synchronize()
+    assert int(bad) == 0, int(bad)
+
+
 @pytest.mark.parametrize("M,cap", [(73, 128), (96, 128)])
 def test_ring_splits_fit_a_buffer_of_other_rows(M, cap):
     # A workspace sized for 128 rows of down_proj holds fewer partials than the
