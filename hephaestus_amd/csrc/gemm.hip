@@ -2,10 +2,11 @@
 //
 // Replaces the reference's prefill kernel wmma_gemm_kernel_v3a_fp8
 // (src/hephaestus/wmma_gfx12.mojo:756-888: 64x64 tile, BK=16, single LDS
-// buffer, two barriers per 16-wide K step, rank-1 scale epilogue). Two
-// kernels: the large-M BMx256 DMA kernel further down (every M while the
-// operands' byte offsets fit 32 bits), and first the 128x128 kernel for
-// larger operands:
+// buffer, two barriers per 16-wide K step, rank-1 scale epilogue). Three
+// families, chosen by gemm_plan below: the large DMA-staged tiles of gemm_big.h
+// and the ring tiles of gemm_ring.h (33 to 1023 rows) while the operands' byte
+// offsets fit 32 bits, and first here the 128x128 kernel for larger operands
+// and for K % 128 != 0:
 //   * 128x128 output tile per 256-thread workgroup, 2x2 waves of 64x64,
 //     each wave 4x4 v_mfma_f32_16x16x128_f8f6f4 per 128-wide K chunk;
 //   * K advances one 128-wide chunk per step, which is exactly one
@@ -334,10 +335,10 @@ static double gemm_estimate(int M, int N, int K, const TileCost& tc, int s, long
 // The ring tiles (gemm_ring.h) and their cost: with n workgroups on the fullest
 // CU, KC chunks each and weights streamed at 5 TB/s at best,
 //     max(2 + n g + KC max(c1, n c), 3 + N K / 5e6) us,
-// a split's reduction 2.5 us and its partials at 4 TB/s (c1 a chunk's latency
-// alone on the CU, c its share of it; fitted to 1230 MI355X times at 47 shapes,
-// M 33 .. 1000, N 1024 .. 19456, K 1024 .. 9728, 1 .. 8 splits, weights from
-// HBM).
+// a split's reduction 2.5 us and its partials at 4 TB/s (c1 stands for a chunk's
+// latency alone on the CU, c for its share of it: coefficients fitted together to
+// 1230 MI355X times at 47 shapes, M 33 .. 1000, N 1024 .. 19456, K 1024 .. 9728,
+// 1 .. 8 splits, weights from HBM).
 struct RingCost {
     int bm, bn;
     double g, c1, c;
@@ -441,11 +442,9 @@ size_t gemm_split_bytes(int M, int N, int K)
 hipError_t launch_fp8_gemm(const Fp8Operands& op, hipStream_t stream,
                            const LaunchTiming& t, const char** name)
 {
-    // The DMA kernel (tiles of 192-320 columns) for every M (N % 16 == 0
-    // keeps every 8-wide output group inside the row), splitting K when its
-    // tiles leave CUs idle; its 32-bit operand offsets need M*K and N*K below
-    // 2^31, else the 128x128 kernel. (Without splits the two run alike below
-    // M = 128; the DMA kernel is 1.3-2x faster from there on, MI355X.)
+    // The DMA-staged tiles for every M (N % 16 == 0 keeps every output group
+    // inside the row), splitting K when they leave CUs idle; their 32-bit operand
+    // offsets need M*K and N*K below 2^31, else the 128x128 kernel.
     const bool small_offsets = (long)op.M * op.K < (1L << 31) && (long)op.N * op.K < (1L << 31);
     const bool force_128 = op.tune.gemm_bm == 1;
     if (small_offsets && !force_128) {

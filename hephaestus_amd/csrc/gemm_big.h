@@ -1,4 +1,5 @@
-// gemm_big.h - the large-M GEMM tile (included by gemm.hip).
+// gemm_big.h - the large-M GEMM tile, E4M3 and bf16 (included by gemm.hip and
+// bf16_gemm.hip).
 #pragma once
 
 #include <type_traits>
@@ -43,7 +44,7 @@ namespace {
 // (nothing varies along K), or unscaled bf16 (a chunk is then 64 elements).
 enum BigType { kBigBlock = 0, kBigChannel = 1, kBigConst = 2, kBigBf16 = 3 };
 
-// Tile BM x BN, BM a multiple of 32 up to 256, BN in {192, 256, 320}: the 8
+// Tile BM x BN, BM a multiple of 32 up to 288, BN in {192, 256, 320}: the 8
 // waves form a 2 x 4 grid of (BM/2) x (BN/4) wave tiles. A smaller tile
 // trades MFMA work per chunk for a tile count that fills the CUs (e.g. 256
 // tiles of 128 x 320 instead of 160 of 256 x 256 at M = 4096, N = 2560).
@@ -115,11 +116,12 @@ __device__ __forceinline__ void pin(f32x4& v) { asm volatile("" : "+v"(v)); }
 }  // namespace
 
 // Epilogue of the large-M kernels: lane l holds C[row r16][cols 4*slice ..
-// +3] of each 16x16 block of its (BM/2) x 64 wave tile, already scaled.
+// +3] of each 16x16 block of its (BM/2) x (BN/4) wave tile, already scaled.
 // K splits store the fp32 partial tile; bf16 output goes through LDS once
 // as bf16 for coalesced 16-byte stores; f32 output or a residual in two
-// f32 passes (the residual added before the one rounding). Every thread of
-// the workgroup calls it; LDS_BYTES of smem are free to reuse.
+// f32 passes (the residual added before the one rounding); the bf16 contraction
+// straight from registers. Every thread of the workgroup calls it; LDS_BYTES of
+// smem are free to reuse.
 template <int SM, int BM, int BN, int LDS_BYTES>
 __device__ __forceinline__ void big_epilogue(const Fp8Operands& op,
                                              f32x4 (&acc)[BM / 32][BN / 64], uint8_t* smem,
@@ -315,7 +317,8 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm256_kernel(Fp8Operands op)
     // instruction per 8 rows, none past the tile) and rows [8 NBP w, 8 NBP (w+1)) of B (NBP = BN / 64
     // instructions); lane i covers row i >> 3 of a block and global
     // piece (i & 7) ^ (row & 7). Rows past M (N) are clamped to the last
-    // row: they feed output rows (columns) that are never stored. Each lane
+    // row, and loaded: they feed output rows (columns) that are never stored
+    // (bf16: nor are the MFMAs of row tiles past M issued). Each lane
     // keeps one 32-bit byte offset per block and operand; chunk j adds the
     // scalar offset 128 * j.
     const rsrc_t rq = make_rsrc(SM == kBigBf16 ? (const void*)op.x : (const void*)op.q);
@@ -432,7 +435,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm256_kernel(Fp8Operands op)
     const int n_parts = a_parts + NBP + (RESCALE && wave * 64 < L_BM ? 1 : 0);
 
     // One 128-wide chunk j held in A stage buf (a compile-time constant)
-    // and B stage bst. The wave's nine DMA instructions (A rows and scales
+    // and B stage bst. The wave's DMA instructions (A rows and scales
     // of chunk j + NS - 1, B rows of chunk j + NB - 1) go out kPer per row
     // tile from the first tile on: issued together right after the barrier,
     // the DMAs of all eight waves stall every wave's instruction issue;
@@ -441,7 +444,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm256_kernel(Fp8Operands op)
     auto chunk = [&](auto bufc, int j, int bst) {
         constexpr int buf = decltype(bufc)::value;
         // with three stages the newest instructions, the next chunk's DMA
-        // (all nine parts, or its four B parts with three B stages), may
+        // (n_parts, or its NBP B parts where only B has three stages), may
         // stay in flight; with two, everything lands
         wait_stage(NB == 3 && j + 1 < je ? (SPLIT_B ? NBP : n_parts) : 0);
         stage_barrier();
