@@ -202,18 +202,18 @@ constexpr Bf16Tile kBf16Tiles[] = {
 // A CU holds two 128 x 128 workgroups of the register-staged kernel, but one
 // of the ring's 128 x 128 or two of its 64 x 64. Where the model takes a ring
 // tile and there are more than 256 tiles of 128 x 128, the register-staged
-// kernel is therefore the faster one for short rows (M > 64, K <= 384: one
-// workgroup's stores hide the other's prologue), and up to 64 rows where its
-// rounds are more than 65 % full and either K <= 2048 or all of it fits one
-// round. MI355X, register-staged against the ring tile: 2528 x 1552 x 128 7.0
-// and 10.0 us, 56 x 59312 x 128 8.8 and 11.9, 65 x 87392 x 256 17.8 and 22.3,
-// 59 x 62000 x 512 17.9 and 21.0, 62 x 52624 x 2560 62.1 and 67.8; on the other
-// side 39 x 80656 x 2048 (rounds 62 % full) 97.5 and 74.3, 64 x 151936 x 2560
-// 189 and 176, 3893 x 816 x 512 12.3 and 10.0. Over 838 drawn shapes (M 33 ..
-// 4096, N 16 .. 152000, K 128 .. 8192) the choice takes 0.77 of the
-// register-staged kernel's time; 9 of them take more than 1.03 (1.10 at worst),
-// 7 with K <= 640 on the tiles of 128 rows and more, which take 0.82 of its
-// time there in the mean. (Of 750 shapes drawn afterwards one takes more, 1.07.)
+// kernel can therefore be the faster one. Its side of the line: short rows
+// (K <= 384, where one workgroup's stores hide the other's prologue), and up to
+// 64 rows one round that is more than 75 % full, or several more than 65 % full
+// against the 128 x 128 tile up to K = 1024. MI355X, register-staged against the
+// ring tile: 2528 x 1552 x 128 7.0 and 10.0 us, 65 x 87392 x 256 17.8 and 22.3, 56
+// x 59312 x 128 8.8 and 11.9, 62 x 52624 x 2560 62.1 and 67.8, 43 x 96416 x 256
+// 17.5 and 20.5. The other side: 157 x 18864 x 256 10.3 and 8.3, one round 67 %
+// full 41 x 43808 x 1408 33.8 and 30.4, several 42 x 141632 x 384 33.5 and 30.0 (64
+// x 64), 64 x 151936 x 2560 189 and 176. Over 838 drawn shapes (M 33 .. 4096, N 16
+// .. 152000, K 128 .. 8192) the choice takes 0.77 of the register-staged kernel's
+// time; 19 of them take more than 1.03 (1.12 at worst). (Of 1300 shapes drawn
+// afterwards four do, 1.06 at worst.)
 int bf16_gemm_tile(int M, int N, int K, bool c_f32)
 {
     const double floor_us =
@@ -238,8 +238,11 @@ int bf16_gemm_tile(int M, int N, int K, bool c_f32)
     const long regs = (long)((M + 127) / 128) * ((N + 127) / 128);
     if (best >= kT128x128 && regs > kPlanCUs) {
         const long slots = 2 * kPlanCUs, rounds = (regs + slots - 1) / slots;
-        const bool full = 100 * regs > 65 * rounds * slots;
-        if (M > 64 ? K <= 384 : full && (K <= 2048 || rounds == 1)) return kReg;
+        const bool wide = best == kT128x128;
+        const bool few = rounds == 1 ? 4 * regs > 3 * slots
+                                     : 20 * regs > 13 * rounds * slots && wide && K <= 1024;
+        if (M > 64 ? K <= 384 && (wide || M <= 128) : few)
+            return kReg;
     }
     return best;
 }

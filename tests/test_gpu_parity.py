@@ -726,8 +726,8 @@ def test_bf16_gemm_every_tile(M, N, K, tile, out, resid):
 
 
 @pytest.mark.parametrize("M,N,K", [
-    (33, 42640, 128), (64, 42752, 640),        # one round of its tiles, two thirds full
-    (35, 109328, 384),                         # two rounds
+    (33, 49168, 128), (64, 49184, 640),        # one round of its tiles, three quarters full
+    (38, 98032, 512),                          # two rounds
     (70, 35296, 128), (2177, 1936, 384)])      # short rows, more than 256 tiles
 @pytest.mark.parametrize("out,resid", [("f32", False), ("bf16", True)])
 def test_bf16_gemm_register_staged(M, N, K, out, resid):
