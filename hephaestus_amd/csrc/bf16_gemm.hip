@@ -212,8 +212,8 @@ constexpr Bf16Tile kBf16Tiles[] = {
 // full 41 x 43808 x 1408 33.8 and 30.4, several 42 x 141632 x 384 33.5 and 30.0 (64
 // x 64), 64 x 151936 x 2560 189 and 176. Over 838 drawn shapes (M 33 .. 4096, N 16
 // .. 152000, K 128 .. 8192) the choice takes 0.77 of the register-staged kernel's
-// time; 19 of them take more than 1.03 (1.12 at worst). (Of 1300 shapes drawn
-// afterwards four do, 1.06 at worst.)
+// time; 19 of them take more than 1.03 (1.12 at worst). (Of 650 shapes drawn
+// afterwards two do, 1.05 at worst.)
 int bf16_gemm_tile(int M, int N, int K, bool c_f32)
 {
     const double floor_us =
